@@ -77,10 +77,8 @@ struct AttnArgs {
   const uint16_t* __restrict__ k;
   const uint16_t* __restrict__ v;
   uint16_t* __restrict__ out;
-  const int32_t* __restrict__ row_ptr;
   const int32_t* __restrict__ col_idx;
   const int32_t* __restrict__ work_ptr;  // [groups + 1]
-  const int32_t* __restrict__ work;
   const int32_t* __restrict__ unit_desc;  // [units][kUnitDescInts], in work order
   int64_t q_hs, k_hs, v_hs, o_hs;  // head strides (elements)
   int32_t q_rs, k_rs, v_rs, o_rs;  // row strides (elements)
@@ -340,10 +338,8 @@ static int launch_bsattn(h3hip_plan p, const View& q, const View& k, const View&
                 static_cast<const uint16_t*>(k.ptr),
                 static_cast<const uint16_t*>(v.ptr),
                 static_cast<uint16_t*>(const_cast<void*>(o.ptr)),
-                p->d_row_ptr,
                 p->d_col_idx,
                 p->d_work_ptr,
-                p->d_work,
                 p->d_unit_desc,
                 q.head_stride,
                 k.head_stride,

@@ -27,7 +27,48 @@ namespace h3hip {
 // XCD runs at one time stay neighbours in its list.
 // Cost of a unit in tile times beyond its tiles (merge, store, first loads),
 // measured on MI355X (band rules: 1.8 us per tile, the rest per unit).
-constexpr double kUnitOverhead = 2.0;
+constexpr int kUnitOverhead = 2;
+
+// Deals a list to `count` workgroups in list order, every unit to the one that
+// is free first (the lowest index of several), and appends each unit's
+// workgroup to wg. Costs are whole numbers of at most max_cost, so all free
+// times lie in a window of max_cost + 1 ticks from the earliest: a ring of
+// buckets, one bit per workgroup, finds the next one in a step or two. For the
+// 10,000 units of 250 x 250 tiles x 40 heads on 256 workgroups build_schedule
+// takes 140 us so and 396 us with a priority queue and a vector per workgroup
+// (one core of the build host). The queue stays for more than 64 workgroups
+// per XCD, which do not fit in a bucket's word.
+static void deal(const std::vector<int32_t>& list, const std::vector<int32_t>& len, int count,
+                 std::vector<int32_t>& wg) {
+  if (count > 64) {
+    std::priority_queue<std::pair<int64_t, int>, std::vector<std::pair<int64_t, int>>,
+                        std::greater<std::pair<int64_t, int>>>
+        free_at;
+    for (int c = 0; c < count; c++) free_at.push({0, c});
+    for (int32_t u : list) {
+      const auto [t, c] = free_at.top();
+      free_at.pop();
+      wg.push_back(c);
+      free_at.push({t + len[u & 0xffff] + kUnitOverhead, c});
+    }
+    return;
+  }
+  int32_t max_cost = 1;
+  for (int32_t u : list) max_cost = std::max(max_cost, len[u & 0xffff] + kUnitOverhead);
+  const int32_t window = max_cost + 1;
+  std::vector<uint64_t> free_at(window, 0);
+  free_at[0] = count == 64 ? ~0ull : (1ull << count) - 1;
+  int32_t now = 0;
+  for (int32_t u : list) {
+    while (free_at[now] == 0) now = now + 1 == window ? 0 : now + 1;
+    const uint64_t c = free_at[now] & (0 - free_at[now]);
+    free_at[now] ^= c;
+    int32_t then = now + len[u & 0xffff] + kUnitOverhead;
+    if (then >= window) then -= window;
+    free_at[then] |= c;
+    wg.push_back(__builtin_ctzll(c));
+  }
+}
 
 int build_schedule(const std::vector<int32_t>& row_ptr, int32_t heads, int32_t groups,
                    std::vector<int32_t>& work_ptr, std::vector<int32_t>& work) {
@@ -60,53 +101,53 @@ int build_schedule(const std::vector<int32_t>& row_ptr, int32_t heads, int32_t g
 
   // Regular rows: one contiguous (head, q-tile) sequence split into ranges that
   // top every XCD up to the same total.
-  std::vector<int32_t> regular;
+  std::vector<int32_t> rows;   // regular rows, the same for every head
   double reg_cost = 0;
-  for (int32_t h = 0; h < heads; h++)
-    for (int32_t i = 0; i < nq; i++)
-      if (len[i] < long_at) {
-        regular.push_back(enc(h, i));
-        reg_cost += len[i] + kUnitOverhead;
-      }
-  double total = reg_cost;
+  for (int32_t i = 0; i < nq; i++)
+    if (len[i] < long_at) {
+      rows.push_back(i);
+      reg_cost += len[i] + kUnitOverhead;
+    }
+  const size_t n_regular = rows.size() * heads;
+  double total = reg_cost * heads;
   for (double c : cost) total += c;
   const double target = total / kXcd;
-  size_t pos = 0;
+  size_t pos = 0, row = 0;
+  int32_t head = 0;
   // Fill the least-loaded XCDs first so ranges stay contiguous per XCD.
   std::vector<int> order(kXcd);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[a] < cost[b]; });
   for (int oi = 0; oi < kXcd; oi++) {
     const int x = order[oi];
-    while (pos < regular.size() && (oi == kXcd - 1 || cost[x] < target)) {
-      const int32_t qt = regular[pos] & 0xffff;
-      lists[x].push_back(regular[pos]);
+    lists[x].reserve(lists[x].size() + n_regular / kXcd * 2);
+    for (; pos < n_regular && (oi == kXcd - 1 || cost[x] < target); pos++) {
+      const int32_t qt = rows[row];
+      lists[x].push_back(enc(head, qt));
       cost[x] += len[qt] + kUnitOverhead;
-      pos++;
+      if (++row == rows.size()) row = 0, head++;
     }
   }
   // Each XCD's list onto its groups / 8 workgroups (workgroup c*8 + x is the
-  // c-th of XCD x).
+  // c-th of XCD x): every unit's workgroup in list order, then a counting sort.
   const int per_xcd = groups / kXcd;
-  std::vector<std::vector<int32_t>> per_wg(groups);
+  std::vector<int32_t> wg;
+  wg.reserve((size_t)heads * nq);
+  work_ptr.assign(groups + 1, 0);
   for (int x = 0; x < kXcd; x++) {
-    std::priority_queue<std::pair<double, int>, std::vector<std::pair<double, int>>,
-                        std::greater<std::pair<double, int>>>
-        free_at;
-    for (int c = 0; c < per_xcd; c++) free_at.push({0.0, c});
-    for (int32_t u : lists[x]) {
-      const auto [t, c] = free_at.top();
-      free_at.pop();
-      per_wg[c * kXcd + x].push_back(u);
-      free_at.push({t + len[u & 0xffff] + kUnitOverhead, c});
+    const size_t first = wg.size();
+    deal(lists[x], len, per_xcd, wg);
+    for (size_t i = first; i < wg.size(); i++) {
+      wg[i] = wg[i] * kXcd + x;
+      work_ptr[wg[i] + 1]++;
     }
   }
-  work_ptr.assign(groups + 1, 0);
-  work.clear();
-  for (int b = 0; b < groups; b++) {
-    work.insert(work.end(), per_wg[b].begin(), per_wg[b].end());
-    work_ptr[b + 1] = (int32_t)work.size();
-  }
+  for (int b = 0; b < groups; b++) work_ptr[b + 1] += work_ptr[b];
+  work.assign(wg.size(), 0);
+  std::vector<int32_t> next(work_ptr.begin(), work_ptr.end() - 1);
+  size_t at = 0;
+  for (int x = 0; x < kXcd; x++)
+    for (int32_t u : lists[x]) work[next[wg[at++]]++] = u;
   // Every (head, q-tile) unit exactly once: a dropped unit would leave its
   // output rows unwritten, a duplicated one would race with itself.
   std::vector<uint8_t> seen((size_t)heads * nq, 0);

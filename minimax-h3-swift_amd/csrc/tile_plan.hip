@@ -143,6 +143,28 @@ __global__ __launch_bounds__(256) void fill_kernel(const uint8_t* bitmap, int32_
   }
 }
 
+// One descriptor (plan.h) per work unit.
+__global__ __launch_bounds__(256) void unit_desc_kernel(const int32_t* work, int32_t units,
+                                                        const int32_t* row_ptr,
+                                                        const int32_t* col_idx, int32_t seq_len,
+                                                        int32_t* desc) {
+  const int32_t u = blockIdx.x * 256 + threadIdx.x;
+  if (u >= units) return;
+  const int32_t unit = work[u], qt = unit & 0xffff;
+  const int32_t beg = row_ptr[qt], n = row_ptr[qt + 1] - beg;
+  int32_t c0 = 0, c1 = 0, c2 = 0, ragged = 0;
+  if (n > 0) {
+    const int32_t* c = col_idx + beg;
+    c0 = c[0];
+    c1 = c[min(1, n - 1)];
+    c2 = c[min(2, n - 1)];
+    ragged = c[n - 1] * H3HIP_TILE + H3HIP_TILE > seq_len ? 1 : 0;
+  }
+  int4* d = reinterpret_cast<int4*>(desc + (size_t)kUnitDescInts * u);
+  d[0] = make_int4(unit, beg, n, c0);
+  d[1] = make_int4(c1, c2, ragged, 0);
+}
+
 // ------------------------------------------------------------ host helpers
 
 static int validate_rule(const h3hip_mask_rule* r) {
@@ -184,7 +206,43 @@ static int validate_rule(const h3hip_mask_rule* r) {
   return H3HIP_OK;
 }
 
-// Small device arrays the rule kernel reads (global columns, landmark flags).
+// flags[0 .. n_flags) = 0, then flags[list[i]] = 1 for i < n_list (list
+// entries are validated on the host). One workgroup; a fill kernel rather
+// than a memset so the clear is an ordinary kernel node.
+__global__ __launch_bounds__(256) void flags_from_list_kernel(uint8_t* flags, int32_t n_flags,
+                                                              const int32_t* list,
+                                                              int32_t n_list) {
+  for (int32_t i = threadIdx.x; i < n_flags; i += 256) flags[i] = 0;
+  __syncthreads();
+  for (int32_t i = threadIdx.x; i < n_list; i += 256) flags[list[i]] = 1;
+}
+
+// The same with the list passed by value in the kernel arguments, so nothing
+// is staged from host memory: the form for short lists, which needs no copy
+// and keeps h3hip_mask_from_rule_noalloc capturable into a HIP graph.
+constexpr int32_t kArgList = 256;
+struct ListArg {
+  int32_t n;
+  int32_t v[kArgList];
+};
+__global__ __launch_bounds__(256) void flags_from_arg_kernel(uint8_t* flags, int32_t n_flags,
+                                                             ListArg list) {
+  for (int32_t i = threadIdx.x; i < n_flags; i += 256) flags[i] = 0;
+  __syncthreads();
+  for (int32_t i = threadIdx.x; i < list.n; i += 256) flags[list.v[i]] = 1;
+}
+
+// flags[0 .. n_flags) on the device from a short host list.
+static int flags_from_arg(uint8_t* flags, int32_t n_flags, const int32_t* list, int32_t n_list,
+                          hipStream_t stream) {
+  ListArg arg{};
+  arg.n = n_list;
+  for (int32_t i = 0; i < n_list; i++) arg.v[i] = list[i];
+  flags_from_arg_kernel<<<1, 256, 0, stream>>>(flags, n_flags, arg);
+  return check_launch("flags_from_arg_kernel");
+}
+
+// The flags the rule kernel reads (global columns or landmark frames).
 struct RuleScratch {
   uint8_t* d = nullptr;
   ~RuleScratch() {
@@ -198,25 +256,23 @@ static int rule_to_device(const h3hip_mask_rule* r, RuleScratch& scratch, RuleDe
   out = RuleDev{r->kind, r->seq_len, r->prefix_len, r->frames, r->height, r->width,
                 r->frame_window, r->spatial_tile_h, r->spatial_tile_w, r->spatial_window,
                 r->band, n_tiles, nullptr, nullptr};
-  std::vector<uint8_t> host;
-  size_t col_off = 0, lm_off = 0;
-  if (r->kind == H3HIP_RULE_BAND) {
-    col_off = host.size();
-    host.resize(host.size() + n_tiles, 0);
-    for (int32_t i = 0; i < r->n_global_cols; i++) host[col_off + r->global_cols[i]] = 1;
+  const bool band = r->kind == H3HIP_RULE_BAND;
+  const bool lattice = r->kind == H3HIP_RULE_LOCAL || r->kind == H3HIP_RULE_AXIAL;
+  if (!band && !(lattice && r->n_landmarks > 0)) return H3HIP_OK;
+  const int32_t n_flags = band ? n_tiles : r->frames;
+  const int32_t* list = band ? r->global_cols : r->landmark_frames;
+  const int32_t n_list = band ? r->n_global_cols : r->n_landmarks;
+  H3_HIP_CHECK(hipMalloc(&scratch.d, n_flags));
+  if (n_list <= kArgList) {
+    const int rc = flags_from_arg(scratch.d, n_flags, list, n_list, stream);
+    if (rc != H3HIP_OK) return rc;
+  } else {
+    std::vector<uint8_t> host(n_flags, 0);
+    for (int32_t i = 0; i < n_list; i++) host[list[i]] = 1;
+    H3_HIP_CHECK(hipMemcpyAsync(scratch.d, host.data(), n_flags, hipMemcpyHostToDevice, stream));
+    H3_HIP_CHECK(hipStreamSynchronize(stream));
   }
-  if ((r->kind == H3HIP_RULE_LOCAL || r->kind == H3HIP_RULE_AXIAL) && r->n_landmarks > 0) {
-    lm_off = host.size();
-    host.resize(host.size() + r->frames, 0);
-    for (int32_t i = 0; i < r->n_landmarks; i++) host[lm_off + r->landmark_frames[i]] = 1;
-  }
-  if (host.empty()) return H3HIP_OK;
-  H3_HIP_CHECK(hipMalloc(&scratch.d, host.size()));
-  H3_HIP_CHECK(hipMemcpyAsync(scratch.d, host.data(), host.size(), hipMemcpyHostToDevice, stream));
-  H3_HIP_CHECK(hipStreamSynchronize(stream));
-  if (r->kind == H3HIP_RULE_BAND) out.col_global = scratch.d + col_off;
-  if ((r->kind == H3HIP_RULE_LOCAL || r->kind == H3HIP_RULE_AXIAL) && r->n_landmarks > 0)
-    out.frame_landmark = scratch.d + lm_off;
+  (band ? out.col_global : out.frame_landmark) = scratch.d;
   return H3HIP_OK;
 }
 
@@ -268,45 +324,14 @@ static int scratch_on_current_device(uint8_t** out) {
   return H3HIP_OK;
 }
 
-// flags[0 .. n_flags) = 0, then flags[list[i]] = 1 for i < n_list (list
-// entries are validated on the host). One workgroup; a fill kernel rather
-// than a memset so the clear is an ordinary kernel node.
-__global__ __launch_bounds__(256) void flags_from_list_kernel(uint8_t* flags, int32_t n_flags,
-                                                              const int32_t* list,
-                                                              int32_t n_list) {
-  for (int32_t i = threadIdx.x; i < n_flags; i += 256) flags[i] = 0;
-  __syncthreads();
-  for (int32_t i = threadIdx.x; i < n_list; i += 256) flags[list[i]] = 1;
-}
-
-// The same with the list passed by value in the kernel arguments, so nothing
-// is staged from host memory: the form h3hip_mask_from_rule_noalloc uses for
-// short lists, which keeps it capturable into a HIP graph.
-constexpr int32_t kArgList = 256;
-struct ListArg {
-  int32_t n;
-  int32_t v[kArgList];
-};
-__global__ __launch_bounds__(256) void flags_from_arg_kernel(uint8_t* flags, int32_t n_flags,
-                                                             ListArg list) {
-  for (int32_t i = threadIdx.x; i < n_flags; i += 256) flags[i] = 0;
-  __syncthreads();
-  for (int32_t i = threadIdx.x; i < list.n; i += 256) flags[list.v[i]] = 1;
-}
-
-static int csr_on_device(const uint8_t* d_bitmap, int32_t nq, int32_t nk, int32_t* d_row_ptr,
-                         hipStream_t stream, int64_t* nnz) {
+// row_ptr[0 .. nq] of the bitmap, on the device.
+static int launch_row_ptr(const uint8_t* d_bitmap, int32_t nq, int32_t nk, int32_t* d_row_ptr,
+                          hipStream_t stream) {
   row_count_kernel<<<nq, 256, 0, stream>>>(d_bitmap, nk, d_row_ptr);
-  int rc = check_launch("row_count_kernel");
+  const int rc = check_launch("row_count_kernel");
   if (rc) return rc;
   scan_kernel<<<1, 256, 0, stream>>>(d_row_ptr, nq);
-  rc = check_launch("scan_kernel");
-  if (rc) return rc;
-  int32_t last = 0;
-  H3_HIP_CHECK(hipMemcpyAsync(&last, d_row_ptr + nq, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
-  H3_HIP_CHECK(hipStreamSynchronize(stream));
-  *nnz = last;
-  return H3HIP_OK;
+  return check_launch("scan_kernel");
 }
 
 }  // namespace h3hip
@@ -385,12 +410,8 @@ int h3hip_mask_from_rule_noalloc(const h3hip_mask_rule* rule, uint8_t* d_bitmap,
     if (rc) return rc;
     uint8_t* flags = band ? sp : sp + kScratchFlags;
     if (by_value) {
-      ListArg arg{};
-      arg.n = n_list;
-      const int32_t* src = band ? rule->global_cols : rule->landmark_frames;
-      for (int32_t i = 0; i < n_list; i++) arg.v[i] = src[i];
-      flags_from_arg_kernel<<<1, 256, 0, st>>>(flags, n_flags, arg);
-      rc = check_launch("flags_from_arg_kernel");
+      rc = flags_from_arg(flags, n_flags, band ? rule->global_cols : rule->landmark_frames,
+                          n_list, st);
     } else {
       int32_t* list = reinterpret_cast<int32_t*>(sp + 2 * kScratchFlags);
       H3_HIP_CHECK(hipMemcpyAsync(list, band ? rule->global_cols : rule->landmark_frames,
@@ -416,8 +437,12 @@ int h3hip_tiles_from_mask(const uint8_t* d_bitmap, int32_t nq, int32_t nk, int32
   H3_REQUIRE(d_bitmap && d_row_ptr && nnz, H3HIP_EINVAL, "NULL argument");
   H3_REQUIRE(nq > 0 && nk > 0, H3HIP_EINVAL, "nq and nk must be positive");
   hipStream_t s = as_stream(stream);
-  int rc = csr_on_device(d_bitmap, nq, nk, d_row_ptr, s, nnz);
+  const int rc = launch_row_ptr(d_bitmap, nq, nk, d_row_ptr, s);
   if (rc) return rc;
+  int32_t last = 0;
+  H3_HIP_CHECK(hipMemcpyAsync(&last, d_row_ptr + nq, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  H3_HIP_CHECK(hipStreamSynchronize(s));
+  *nnz = last;
   H3_REQUIRE(col_capacity >= *nnz, H3HIP_EINVAL, "col_capacity %lld < nnz %lld",
              (long long)col_capacity, (long long)*nnz);
   if (*nnz == 0) return H3HIP_OK;
@@ -460,9 +485,16 @@ int h3hip_plan_create(const h3hip_mask_rule* rule, int32_t heads, const h3hip_po
   RuleScratch scratch;
   rc = launch_mask(rule, d_bitmap, s, scratch);
   if (rc) return fail(rc);
-  int64_t nnz = 0;
-  rc = csr_on_device(d_bitmap, n, n, p->d_row_ptr, s, &nnz);
+  rc = launch_row_ptr(d_bitmap, n, n, p->d_row_ptr, s);
   if (rc) return fail(rc);
+  p->row_ptr.resize(n + 1);
+  if (hipMemcpyAsync(p->row_ptr.data(), p->d_row_ptr, sizeof(int32_t) * (n + 1),
+                     hipMemcpyDeviceToHost, s) != hipSuccess ||
+      hipStreamSynchronize(s) != hipSuccess) {
+    set_error("copying the tile lists back failed");
+    return fail(H3HIP_EHIP);
+  }
+  const int64_t nnz = p->row_ptr[n];
   p->nnz = nnz;
   if (hipMalloc(&p->d_col_idx, sizeof(int32_t) * std::max<int64_t>(nnz, 1)) != hipSuccess) {
     set_error("device allocation for %lld tile indices failed", (long long)nnz);
@@ -473,20 +505,10 @@ int h3hip_plan_create(const h3hip_mask_rule* rule, int32_t heads, const h3hip_po
     rc = check_launch("fill_kernel");
     if (rc) return fail(rc);
   }
-  p->row_ptr.resize(n + 1);
-  p->col_idx.resize(nnz);
-  if (hipMemcpyAsync(p->row_ptr.data(), p->d_row_ptr, sizeof(int32_t) * (n + 1),
-                     hipMemcpyDeviceToHost, s) != hipSuccess ||
-      (nnz > 0 && hipMemcpyAsync(p->col_idx.data(), p->d_col_idx, sizeof(int32_t) * nnz,
-                                 hipMemcpyDeviceToHost, s) != hipSuccess) ||
-      hipStreamSynchronize(s) != hipSuccess) {
-    set_error("copying the tile lists back failed");
-    return fail(H3HIP_EHIP);
-  }
-  (void)hipFree(d_bitmap);
-  d_bitmap = nullptr;
 
-  // One persistent attention workgroup per CU, a whole number per XCD.
+  // One persistent attention workgroup per CU, a whole number per XCD. The
+  // schedule needs the row lengths only: the host builds it while the columns
+  // are filled, and the unit descriptors are made on the device.
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
@@ -496,41 +518,38 @@ int h3hip_plan_create(const h3hip_mask_rule* rule, int32_t heads, const h3hip_po
   p->groups = std::max(8, cus / 8 * 8);
   rc = build_schedule(p->row_ptr, heads, p->groups, p->work_ptr, p->work);
   if (rc) return fail(rc);
-  p->unit_desc.assign(p->work.size() * kUnitDescInts, 0);
-  for (size_t u = 0; u < p->work.size(); u++) {
-    const int32_t unit = p->work[u], qt = unit & 0xffff;
-    const int32_t beg = p->row_ptr[qt], n = p->row_ptr[qt + 1] - beg;
-    int32_t* d = &p->unit_desc[kUnitDescInts * u];
-    d[0] = unit;
-    d[1] = beg;
-    d[2] = n;
-    if (n > 0) {
-      const int32_t* c = &p->col_idx[beg];
-      d[3] = c[0];
-      d[4] = c[n > 1 ? 1 : 0];
-      d[5] = c[n > 2 ? 2 : n - 1];
-      d[6] = (int64_t)c[n - 1] * 128 + 128 > p->seq_len ? 1 : 0;
-    }
-  }
-  const size_t desc_bytes = sizeof(int32_t) * std::max<size_t>(p->unit_desc.size(), 1);
-  if (hipMalloc(&p->d_work_ptr, sizeof(int32_t) * p->work_ptr.size()) != hipSuccess ||
-      hipMalloc(&p->d_work, sizeof(int32_t) * std::max<size_t>(p->work.size(), 1)) != hipSuccess ||
-      hipMalloc(&p->d_unit_desc, desc_bytes) != hipSuccess) {
+  const size_t units = p->work.size();
+  auto aligned = [](size_t ints) { return (ints + kListAlign - 1) / kListAlign * kListAlign; };
+  const size_t work_at = aligned(p->work_ptr.size()), desc_at = work_at + aligned(units);
+  std::vector<int32_t> lists(desc_at, 0);
+  std::copy(p->work_ptr.begin(), p->work_ptr.end(), lists.begin());
+  std::copy(p->work.begin(), p->work.end(), lists.begin() + work_at);
+  if (hipMalloc(&p->d_lists, sizeof(int32_t) * (desc_at + kUnitDescInts * units)) !=
+      hipSuccess) {
     set_error("device allocation for the work list failed");
     return fail(H3HIP_ENOMEM);
   }
-  if (hipMemcpyAsync(p->d_work_ptr, p->work_ptr.data(), sizeof(int32_t) * p->work_ptr.size(),
-                     hipMemcpyHostToDevice, s) != hipSuccess ||
-      (!p->work.empty() &&
-       (hipMemcpyAsync(p->d_work, p->work.data(), sizeof(int32_t) * p->work.size(),
-                       hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(p->d_unit_desc, p->unit_desc.data(),
-                       sizeof(int32_t) * p->unit_desc.size(), hipMemcpyHostToDevice,
-                       s) != hipSuccess)) ||
-      hipStreamSynchronize(s) != hipSuccess) {
+  p->d_work_ptr = p->d_lists;
+  p->d_unit_desc = p->d_lists + desc_at;
+  if (hipMemcpyAsync(p->d_lists, lists.data(), sizeof(int32_t) * desc_at, hipMemcpyHostToDevice,
+                     s) != hipSuccess) {
     set_error("uploading the work list failed");
     return fail(H3HIP_EHIP);
   }
+  unit_desc_kernel<<<(unsigned)((units + 255) / 256), 256, 0, s>>>(
+      p->d_lists + work_at, (int32_t)units, p->d_row_ptr, p->d_col_idx, p->seq_len,
+      p->d_unit_desc);
+  rc = check_launch("unit_desc_kernel");
+  if (rc) return fail(rc);
+  p->col_idx.resize(nnz);
+  if ((nnz > 0 && hipMemcpyAsync(p->col_idx.data(), p->d_col_idx, sizeof(int32_t) * nnz,
+                                 hipMemcpyDeviceToHost, s) != hipSuccess) ||
+      hipStreamSynchronize(s) != hipSuccess) {
+    set_error("copying the tile lists back failed");
+    return fail(H3HIP_EHIP);
+  }
+  (void)hipFree(d_bitmap);
+  d_bitmap = nullptr;
   *out = p;
   return H3HIP_OK;
 }
@@ -539,9 +558,7 @@ int h3hip_plan_destroy(h3hip_plan p) {
   if (!p) return H3HIP_OK;
   if (p->d_row_ptr) (void)hipFree(p->d_row_ptr);
   if (p->d_col_idx) (void)hipFree(p->d_col_idx);
-  if (p->d_work) (void)hipFree(p->d_work);
-  if (p->d_work_ptr) (void)hipFree(p->d_work_ptr);
-  if (p->d_unit_desc) (void)hipFree(p->d_unit_desc);
+  if (p->d_lists) (void)hipFree(p->d_lists);
   delete p;
   return H3HIP_OK;
 }

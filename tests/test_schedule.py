@@ -59,3 +59,23 @@ def test_refusals(h3):
         h3.schedule(np.array([0, 1], dtype=np.int32), 2, 12)        # groups % 8
     with pytest.raises(h3.H3HIPError):
         h3.schedule(np.array([1, 2], dtype=np.int32), 2, 8)         # row_ptr[0] != 0
+
+
+@pytest.mark.parametrize("groups", [8, 504, 512, 520, 1024])
+def test_dealt_to_the_workgroup_free_first(h3, groups):
+    """Both ways of dealing (a ring of buckets up to 64 workgroups per XCD, a
+    queue above): each XCD's units, in the order they are dealt, go to the
+    workgroup with the least cost so far, the lowest index of several."""
+    rng = np.random.default_rng(groups)
+    n, heads = 61, 30
+    length = np.where(rng.random(n) < 0.1, n, rng.integers(0, 9, n))
+    row_ptr = np.concatenate([[0], np.cumsum(length)]).astype(np.int32)
+    work_ptr, work = h3.schedule(row_ptr, heads, groups)
+    for x in range(8):
+        wgs = [list(work[work_ptr[b]:work_ptr[b + 1]]) for b in range(x, groups, 8)]
+        free, left = [0] * len(wgs), sum(map(len, wgs))
+        while left:
+            c = min(range(len(wgs)), key=lambda i: (free[i], i))
+            assert wgs[c], (x, c)      # the first free workgroup has the next unit
+            free[c] += int(length[wgs[c].pop(0) & 0xFFFF]) + 2
+            left -= 1
