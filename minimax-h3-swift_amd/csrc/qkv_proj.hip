@@ -40,27 +40,10 @@
 
 #include "common.h"
 #include "norm_rope.h"
+#include "proj.h"
 #include "tile_order.h"
 
 namespace h3hip {
-
-struct ProjArgs {
-  const uint16_t* __restrict__ x;        // [seq_len, hidden], row stride ldx
-  const uint16_t* __restrict__ w;        // [3 * heads * 128, hidden], row stride ldw
-  const uint16_t* __restrict__ q_gamma;  // [128]
-  const uint16_t* __restrict__ k_gamma;
-  const void* __restrict__ table;        // [seq_len, rot/2, 2, 2]: bf16 (REFERENCE) or fp32
-  uint16_t* __restrict__ q_out;          // [heads, seq_pad, 128]
-  uint16_t* __restrict__ k_out;
-  uint16_t* __restrict__ v_out;
-  int64_t ldx, ldw;
-  float eps;
-  int32_t hidden, rot, seq_len, seq_pad, heads, tiles_m;
-  // Out-projection mode: n_out output channels, written token-major into
-  // q_out with row stride ldo.
-  int32_t n_out;
-  int64_t ldo;
-};
 
 constexpr int kPM = 256;                  // tokens per workgroup
 constexpr int kPN = 256;                  // output channels per workgroup
@@ -87,18 +70,6 @@ constexpr int kPBufferWord3 = 0x00020000;
 static_assert(kMfmaSub == 2 * kLoadsStep, "one load per two MFMAs of the second sub-step");
 
 typedef int i32x4p __attribute__((ext_vector_type(4)));
-
-// 16-byte chunk c of the 128-byte operand row r sits at c ^ ((r >> 1) & 7):
-// the 16 rows of a 16-lane read phase cover both row parities x 8 chunk
-// positions. Rows 16 apart share the swizzle.
-__device__ __forceinline__ int p_swz(int r) { return (r >> 1) & 7; }
-
-// 16-byte chunk c of the 256-byte epilogue row r sits at c ^ e_swz(r): the
-// 16 rows one accumulator write covers hit 16 distinct positions (every 8-byte
-// slot of a bank window once per 32 lanes), and rows r, r ^ 1 map the chunks
-// 0..7 onto complementary halves, so the 2 rows x 8 lanes of a 16-lane read
-// phase are conflict-free.
-__device__ __forceinline__ int e_swz(int r) { return ((r & 1) << 3) | ((r >> 1) & 7); }
 
 __device__ __forceinline__ i32x4p proj_rsrc(const void* base, uint32_t bytes) {
   const uint64_t b = reinterpret_cast<uint64_t>(base);
@@ -428,6 +399,9 @@ extern "C" int h3hip_qkv_proj(const void* x, int64_t ldx, const void* w, int64_t
              static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(k_out),
              static_cast<uint16_t*>(v_out), ldx, ldw, eps, hidden, rot, seq_len, seq_pad, heads,
              tiles_m, 0, 0};
+  const ProjTile tile = pick_proj_tile(seq_pad, 3 * heads * kHD, hidden, !plain);
+  if (tile != ProjTile::kEightWave)
+    return launch_proj_gemm(a, tile, rounding, plain, false, as_stream(stream));
   // 8 x the longest XCD list of the tile order (a few empty workgroups when
   // the lists differ in length).
   const TileOrder order{tiles_m, 3 * heads * kHD / kPN};
@@ -474,6 +448,9 @@ extern "C" int h3hip_out_proj(const void* x, int64_t ldx, const void* w, int64_t
   ProjArgs a{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), nullptr, nullptr,
              nullptr, static_cast<uint16_t*>(y), nullptr, nullptr, ldx, ldw, 0.f, in_features,
              128, seq_len, tiles_m * kPM, 1, tiles_m, out_features, ldy};
+  const ProjTile tile = pick_proj_tile(seq_len, out_features, in_features, false);
+  if (tile != ProjTile::kEightWave)
+    return launch_proj_gemm(a, tile, H3HIP_ROUND_REFERENCE, true, true, as_stream(stream));
   const TileOrder order{tiles_m, out_features / kPN};
   int longest = 0;
   for (int xcd = 0; xcd < kXcds; xcd++) longest = std::max(longest, order.length(xcd));
