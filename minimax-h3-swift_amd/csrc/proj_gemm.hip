@@ -48,27 +48,37 @@ __device__ __forceinline__ uint32_t uniform(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
 
-template <int kNA, int kMB>
-struct Shape;
-template <>
-struct Shape<8, 8> {
-  static constexpr int kLds = H3_GEMM_LDS_256x256, kXAt = H3_GEMM_X_AT_256x256,
-                       kBases = H3_GEMM_BASES_256x256;
-};
-template <>
-struct Shape<8, 4> {
-  static constexpr int kLds = H3_GEMM_LDS_256x128, kXAt = H3_GEMM_X_AT_256x128,
-                       kBases = H3_GEMM_BASES_256x128;
-};
-template <>
-struct Shape<4, 4> {
-  static constexpr int kLds = H3_GEMM_LDS_128x128, kXAt = H3_GEMM_X_AT_128x128,
-                       kBases = H3_GEMM_BASES_128x128;
-};
-
 #define H3_SCALARS                                                                          \
   [x_lo] "s"(x_lo), [x_hi] "s"(x_hi), [x_rec] "s"(x_rec), [w_lo] "s"(w_lo), [w_hi] "s"(w_hi), \
       [w_rec] "s"(w_rec), [steps] "s"(steps), [m0x] "s"(m0x), [m0w] "s"(m0w)
+
+// One tile shape: its LDS and its reduction loop, from lane offsets and scalars
+// to accumulators.
+template <int kNA, int kMB>
+struct Shape;
+#define H3_SHAPE(NA, MB, NAME)                                                               \
+  template <>                                                                                \
+  struct Shape<NA, MB> {                                                                     \
+    static constexpr int kLds = H3_GEMM_LDS_##NAME, kXAt = H3_GEMM_X_AT_##NAME,              \
+                         kBases = H3_GEMM_BASES_##NAME;                                      \
+    static __device__ __forceinline__ void reduce(f32x32 (&c)[NA * MB / 8], const int* ra,   \
+                                                  const int* rb, const int* xv, const int* wv, \
+                                                  uint32_t x_lo, uint32_t x_hi, uint32_t x_rec, \
+                                                  uint32_t w_lo, uint32_t w_hi, uint32_t w_rec, \
+                                                  uint32_t steps, uint32_t m0x, uint32_t m0w) { \
+      asm volatile(H3_GEMM_LOOP_##NAME                                                       \
+                   : H3_GEMM_OUT_##NAME(c)                                                   \
+                   : H3_GEMM_IN_##NAME(ra, rb, xv, wv), H3_SCALARS                           \
+                   : H3_GEMM_CLOBBERS_##NAME);                                               \
+    }                                                                                        \
+  };
+H3_SHAPE(8, 8, 256x256)
+H3_SHAPE(8, 7, 256x224)
+H3_SHAPE(8, 6, 256x192)
+H3_SHAPE(8, 5, 256x160)
+H3_SHAPE(8, 4, 256x128)
+H3_SHAPE(4, 4, 128x128)
+H3_SHAPE(4, 2, 128x64)
 
 // The tile's epilogue. Accumulator (na, mb) of lane (g, lr): channels
 // 16 (kNA wc + na) + 4g .. +3 of token 16 (kMB wt + mb) + lr. kHl = rot / 16
@@ -154,13 +164,15 @@ __device__ __forceinline__ void finish_tile(const ProjArgs& a, uint16_t* lds,
       *reinterpret_cast<u32x4*>(dst + 8 * chunk_b) = ob;
     }
   };
-  // A wave's rows lie in one 128-row block, so they are all below seq_pad or
-  // all past it.
-  static_assert(128 % kRows == 0, "");
-  if (!kOut && m0 + row0 >= a.seq_pad) return;
+  // Passes of 8 rows; head-major rows end at seq_pad, a multiple of 8.
+  const int passes = kOut ? kRows / 8 : min(kRows, max(a.seq_pad - m0 - row0, 0)) / 8;
   auto finish_rows = [&](auto whole, auto rotated) __attribute__((always_inline)) {
+    if constexpr (decltype(whole)::value) {
 #pragma unroll 2
-    for (int pass = 0; pass < kRows / 8; pass++) finish_row(row0 + 8 * pass + rg, whole, rotated);
+      for (int pass = 0; pass < kRows / 8; pass++) finish_row(row0 + 8 * pass + rg, whole, rotated);
+    } else {
+      for (int pass = 0; pass < passes; pass++) finish_row(row0 + 8 * pass + rg, whole, rotated);
+    }
   };
   const bool whole = m0 + row0 + kRows <= a.seq_len;
   if constexpr (!kPlain && !kOut) {
@@ -225,24 +237,7 @@ __global__ __launch_bounds__(kThreads, 1) void proj_gemm_kernel(ProjArgs a) {
   const uint32_t m0w = uniform(lds_base + 1024u * kNA * wave);
   const uint32_t m0x = uniform(lds_base + 1024u * kMB * wave);
   f32x32 c[kNA * kMB / 8];
-  if constexpr (kNA == 8 && kMB == 8)
-    asm volatile(H3_GEMM_LOOP_256x256
-                 : "=&{a[0:31]}"(c[0]), "=&{a[32:63]}"(c[1]), "=&{a[64:95]}"(c[2]),
-                   "=&{a[96:127]}"(c[3]), "=&{a[128:159]}"(c[4]), "=&{a[160:191]}"(c[5]),
-                   "=&{a[192:223]}"(c[6]), "=&{a[224:255]}"(c[7])
-                 : H3_GEMM_IN_256x256(ra, rb, xv, wv), H3_SCALARS
-                 : H3_GEMM_CLOBBERS_256x256);
-  else if constexpr (kNA == 8)
-    asm volatile(H3_GEMM_LOOP_256x128
-                 : "=&{a[0:31]}"(c[0]), "=&{a[32:63]}"(c[1]), "=&{a[64:95]}"(c[2]),
-                   "=&{a[96:127]}"(c[3])
-                 : H3_GEMM_IN_256x128(ra, rb, xv, wv), H3_SCALARS
-                 : H3_GEMM_CLOBBERS_256x128);
-  else
-    asm volatile(H3_GEMM_LOOP_128x128
-                 : "=&{a[0:31]}"(c[0]), "=&{a[32:63]}"(c[1])
-                 : H3_GEMM_IN_128x128(ra, rb, xv, wv), H3_SCALARS
-                 : H3_GEMM_CLOBBERS_128x128);
+  S::reduce(c, ra, rb, xv, wv, x_lo, x_hi, x_rec, w_lo, w_hi, w_rec, steps, m0x, m0w);
 
   // The lane again, from the lane counter: kept from before the loop it would
   // be spilled across it.
@@ -280,8 +275,12 @@ int launch_proj_gemm(const ProjArgs& a, ProjTile tile, int32_t rounding, bool pl
                      hipStream_t stream) {
   switch (tile) {
     case ProjTile::k256x256: return launch<8, 8>(a, rounding, plain, out, stream);
+    case ProjTile::k256x224: return launch<8, 7>(a, rounding, plain, out, stream);
+    case ProjTile::k256x192: return launch<8, 6>(a, rounding, plain, out, stream);
+    case ProjTile::k256x160: return launch<8, 5>(a, rounding, plain, out, stream);
     case ProjTile::k256x128: return launch<8, 4>(a, rounding, plain, out, stream);
-    default: return launch<4, 4>(a, rounding, plain, out, stream);
+    case ProjTile::k128x128: return launch<4, 4>(a, rounding, plain, out, stream);
+    default: return launch<4, 2>(a, rounding, plain, out, stream);
   }
 }
 

@@ -18,12 +18,15 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("tile,S,fin,fout,ldx,ldy", [
-    ("256x256", 897, 1088, 15360, None, None),
+    ("256x256", 1000, 1088, 15360, None, None),
+    ("256x224", 801, 1024, 15360, None, None),
+    ("256x192", 700, 1152, 15360, 1160, 15368),
+    ("256x160", 600, 192, 15360, None, None),
     ("256x128", 1001, 192, 5120, 200, 5128),
     ("256x128", 1001, 64, 5120, None, None),
     ("256x128", 897, 320, 5376, None, None),
-    ("128x128", 129, 64, 256, None, 264),
-    ("128x128", 300, 448, 512, 456, None),
+    ("128x128", 400, 448, 5120, 456, None),
+    ("128x64", 129, 64, 256, None, 264),
 ])
 def test_out_proj(tile, S, fin, fout, ldx, ldy):
     from h3hip import ops
@@ -37,14 +40,15 @@ def test_out_proj(tile, S, fin, fout, ldx, ldy):
 
 
 @pytest.mark.parametrize("tile,S,hidden,H,rot,rounding", [
-    ("256x256", 641, 1536, 40, 128, 0),
-    ("256x256", 700, 1600, 40, 96, 1),
-    ("256x128", 1000, 64, 14, 96, 0),
-    ("256x128", 900, 128, 14, 128, 1),
-    ("256x128", 1001, 256, 14, 128, 0),
-    ("128x128", 130, 704, 4, 128, 0),
-    ("128x128", 256, 64, 2, 96, 1),
-] + [("128x128", 200, 64 * k, 2, 128, 0) for k in range(2, 8)])
+    ("256x256", 1000, 1536, 40, 128, 0),
+    ("256x224", 1270, 1600, 56, 96, 0),    # seq_pad 1,280 ends inside the sixth tile
+    ("256x192", 1000, 1536, 56, 96, 1),    # seq_pad 1,024 ends inside the sixth tile
+    ("256x160", 1100, 1536, 40, 128, 0),   # seq_pad 1,152 ends inside the eighth tile
+    ("256x160", 600, 128, 40, 128, 1),
+    ("256x128", 1250, 256, 14, 128, 0),
+    ("128x128", 1000, 704, 6, 96, 0),
+    ("128x64", 256, 64, 2, 96, 1),
+] + [("128x64", 200, 64 * k, 2, 128, 0) for k in range(2, 8)])
 def test_qkv(orc, tile, S, hidden, H, rot, rounding):
     note(f"qkv tile {tile} S={S} hidden={hidden} H={H} rot={rot} rounding={rounding}")
     x, w, plain, fused, (want_q, want_k) = _run(orc, S, hidden, H, rot, rounding)

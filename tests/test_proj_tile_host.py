@@ -10,21 +10,26 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "minimax-h3-swift_amd", "csrc")
-TILES = ["8wave", "256x256", "256x128", "128x128"]
+TILES = ["8wave", "256x256", "256x224", "256x192", "256x160", "256x128", "128x128", "128x64"]
 
 # (tile, tokens, channels, reduction, with norm and RoPE)
 CASES = [
     ("256x256", 31885, 5120, 5120, 0), ("256x256", 32000, 15360, 5120, 1),
-    ("256x256", 768, 15360, 1536, 1), ("8wave", 768, 15360, 1472, 1),
-    ("256x256", 896, 15360, 1024, 0), ("8wave", 896, 15360, 960, 0),
-    ("256x128", 917, 5120, 5120, 0), ("256x128", 1152, 21504, 5376, 1),
-    ("256x128", 4096, 5120, 5120, 0), ("8wave", 4096, 5120, 512, 0),
-    ("128x128", 300, 5120, 5120, 0), ("128x128", 1, 256, 64, 0),
+    ("256x128", 917, 5120, 5120, 0), ("256x192", 1152, 21504, 5376, 1),
+    ("256x192", 4096, 5120, 5120, 0), ("8wave", 4096, 5120, 512, 0),
+    ("256x192", 2048, 5120, 5120, 0), ("8wave", 2048, 5120, 960, 0),
+    ("128x64", 300, 5120, 5120, 0), ("128x64", 1, 256, 64, 0),
+    ("256x192", 768, 15360, 1536, 1), ("8wave", 768, 15360, 1472, 1),
     # test_gpu_proj_tiles.py
-    ("256x256", 768, 15360, 1536, 1), ("256x256", 897, 15360, 1088, 0),
-    ("256x128", 1001, 5120, 192, 0), ("256x128", 1024, 5376, 64, 1),
-    ("256x128", 897, 5376, 320, 0), ("128x128", 256, 1536, 704, 1),
-    ("128x128", 129, 256, 64, 0),
+    ("256x256", 1000, 15360, 1088, 0), ("256x224", 801, 15360, 1024, 0),
+    ("256x192", 700, 15360, 1152, 0), ("256x160", 600, 15360, 192, 0),
+    ("256x128", 1001, 5120, 192, 0), ("256x128", 1001, 5120, 64, 0),
+    ("256x128", 897, 5376, 320, 0), ("128x128", 400, 5120, 448, 0),
+    ("128x64", 129, 256, 64, 0),
+    ("256x256", 1024, 15360, 1536, 1), ("256x224", 1280, 21504, 1600, 1),
+    ("256x192", 1024, 21504, 1536, 1), ("256x160", 1152, 15360, 1536, 1),
+    ("256x160", 640, 15360, 128, 1), ("256x128", 1280, 5376, 256, 1),
+    ("128x128", 1024, 2304, 704, 1), ("128x64", 256, 768, 64, 1),
 ]
 
 HARNESS = r"""
@@ -65,8 +70,7 @@ def test_few_steps_take_small_tiles_only_for_one_round(pick):
     cases = [(t, n, h, f) for t in (1, 130, 700, 2000, 9000) for n in (256, 1536, 5120, 15360)
              for h in (64, 512, 960) for f in (0, 1)]
     for (t, n, h, f), tile in zip(cases, pick(cases)):
-        if tile in ("256x128", "128x128"):
-            tm, tn = (128, 256) if tile == "256x128" else (128, 128)
+        if tile != "8wave":
+            tn, tm = map(int, tile.split("x"))
+            assert tm <= 160
             assert -(-t // tm) * (n // tn) <= 256, (t, n, h, f, tile)
-        else:
-            assert tile == "8wave"
