@@ -44,8 +44,8 @@ OUT = os.path.join(HERE, "gemm_loop.inc")
 
 # name (channels x tokens): (NA, MB, RW, RX); 160 KiB of LDS hold the rings
 VARIANTS = {"256x256": (8, 8, 3, 2), "256x224": (8, 7, 3, 2), "256x192": (8, 6, 3, 2),
-            "256x160": (8, 5, 3, 3), "256x128": (8, 4, 3, 3), "128x128": (4, 4, 5, 5),
-            "128x64": (4, 2, 5, 5)}
+            "256x160": (8, 5, 3, 3), "256x128": (8, 4, 3, 3), "128x192": (4, 6, 4, 4),
+            "128x160": (4, 5, 4, 4), "128x128": (4, 4, 5, 5), "128x64": (4, 2, 5, 5)}
 WAVES = 4
 ROW = 128                 # bytes of a row of one step
 
@@ -238,7 +238,7 @@ def render():
                for arg, at, n in (("RA", g.ra, 2 * g.bases), ("RB", g.rb, 2 * g.bases),
                                   ("XV", g.xv, g.x_loads), ("WV", g.wv, g.w_loads))
                for i in range(n)]
-        acc = [f'"=&{{a[{32 * i}:{32 * i + 31}]}}"(C[{i}])' for i in range(na * mb // 8)]
+        acc = [f'"=&{{a[{32 * i}:{32 * i + 31}]}}"(C[{i}])' for i in range(-(-na * mb // 8))]
         out += [f"// {32 * na} channels x {32 * mb} tokens: {len(lines)} lines.",
                 f"#define H3_GEMM_LDS_{name} {g.lds}",
                 f"#define H3_GEMM_X_AT_{name} {g.x_at}",

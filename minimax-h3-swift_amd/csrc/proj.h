@@ -23,6 +23,7 @@ struct ProjArgs {
   // q_out with row stride ldo.
   int32_t n_out;
   int64_t ldo;
+  int32_t chunk;   // proj_gemm_kernel: token tiles per chunk of its launch order
 };
 
 // 16-byte chunk c of the 128-byte operand row r sits at c ^ ((r >> 1) & 7):

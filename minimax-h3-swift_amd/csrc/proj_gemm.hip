@@ -14,8 +14,9 @@
 // 3.52 against 3.67 ms, out-projection 1.14 against 1.22 ms.
 //
 // Small grids take smaller tiles of the same loop, so that more CUs work: the
-// out-projection of 917 tokens at 5,120 is 80 tiles of 256 x 256 (87 us), or 160
-// of 256 x 128 (52 us); of 300 tokens 40 (85 us), or 120 of 128 x 128 (31 us). All
+// out-projection of 917 tokens at 5,120 is 80 tiles of 256 x 256 (81 us; 87 on
+// eight waves) or 240 of 128 x 160 (42 us), of 300 tokens 40 (80 us) or 200 of 128
+// x 64 (25 us). All
 // shapes add a channel's products in the same order, so their results are the
 // same bits.
 //
@@ -25,7 +26,6 @@
 // code (norm_rope.h) and the render's rotation table. Rows that are complete
 // run without a branch so that two passes overlap: one wave per SIMD has no
 // other to cover its latencies.
-#include <algorithm>
 #include <type_traits>
 
 #include "gemm_loop.inc"
@@ -43,6 +43,9 @@ constexpr int kHead = 128;
 constexpr int kStep = 64;                // reduction per step
 
 typedef float f32x32 __attribute__((ext_vector_type(32)));
+// A wave's accumulators, 8 blocks of 16 x 16 to a vector (the last may be part used).
+template <int kNA, int kMB>
+constexpr int kAccs = (kNA * kMB + 7) / 8;
 
 __device__ __forceinline__ uint32_t uniform(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
@@ -61,7 +64,7 @@ struct Shape;
   struct Shape<NA, MB> {                                                                     \
     static constexpr int kLds = H3_GEMM_LDS_##NAME, kXAt = H3_GEMM_X_AT_##NAME,              \
                          kBases = H3_GEMM_BASES_##NAME;                                      \
-    static __device__ __forceinline__ void reduce(f32x32 (&c)[NA * MB / 8], const int* ra,   \
+    static __device__ __forceinline__ void reduce(f32x32 (&c)[kAccs<NA, MB>], const int* ra,   \
                                                   const int* rb, const int* xv, const int* wv, \
                                                   uint32_t x_lo, uint32_t x_hi, uint32_t x_rec, \
                                                   uint32_t w_lo, uint32_t w_hi, uint32_t w_rec, \
@@ -77,6 +80,8 @@ H3_SHAPE(8, 7, 256x224)
 H3_SHAPE(8, 6, 256x192)
 H3_SHAPE(8, 5, 256x160)
 H3_SHAPE(8, 4, 256x128)
+H3_SHAPE(4, 6, 128x192)
+H3_SHAPE(4, 5, 128x160)
 H3_SHAPE(4, 4, 128x128)
 H3_SHAPE(4, 2, 128x64)
 
@@ -86,7 +91,7 @@ H3_SHAPE(4, 2, 128x64)
 // unchanged; kOut: the out-projection, token-major with row stride ldo.
 template <int kNA, int kMB, int kMode, int kHl, bool kPlain, bool kOut>
 __device__ __forceinline__ void finish_tile(const ProjArgs& a, uint16_t* lds,
-                                            const f32x32 (&c)[kNA * kMB / 8], int wave, int lane,
+                                            const f32x32 (&c)[kAccs<kNA, kMB>], int wave, int lane,
                                             int m0, int n0) {
   constexpr int kTokens = 32 * kMB, kChannels = 32 * kNA;
   const int wc = wave >> 1, wt = wave & 1, lr = lane & 15, g = lane >> 4;
@@ -201,7 +206,7 @@ __global__ __launch_bounds__(kThreads, 1) void proj_gemm_kernel(ProjArgs a) {
   const int wc = wave >> 1, wt = wave & 1;   // channel and token half of the tile
   const int inner = a.heads * kHead;
   const int n_total = kOut ? a.n_out : 3 * inner;
-  const TileOrder order{a.tiles_m, n_total / kChannels};
+  const TileOrder order{a.tiles_m, n_total / kChannels, a.chunk};
   const int xcd = blockIdx.x % kOrderXcds, slot = blockIdx.x / kOrderXcds;
   if (slot >= order.length(xcd)) return;
   const int tile = order.tile(xcd, slot);
@@ -236,7 +241,7 @@ __global__ __launch_bounds__(kThreads, 1) void proj_gemm_kernel(ProjArgs a) {
   const uint32_t steps = uniform((uint32_t)(a.hidden / kStep));
   const uint32_t m0w = uniform(lds_base + 1024u * kNA * wave);
   const uint32_t m0x = uniform(lds_base + 1024u * kMB * wave);
-  f32x32 c[kNA * kMB / 8];
+  f32x32 c[kAccs<kNA, kMB>];
   S::reduce(c, ra, rb, xv, wv, x_lo, x_hi, x_rec, w_lo, w_hi, w_rec, steps, m0x, m0w);
 
   // The lane again, from the lane counter: kept from before the loop it would
@@ -248,11 +253,11 @@ __global__ __launch_bounds__(kThreads, 1) void proj_gemm_kernel(ProjArgs a) {
 
 template <int kNA, int kMB>
 int launch(ProjArgs a, int32_t rounding, bool plain, bool out, hipStream_t st) {
-  a.tiles_m = ((out ? a.seq_len : a.seq_pad) + 32 * kMB - 1) / (32 * kMB);
-  const TileOrder order{a.tiles_m, (out ? a.n_out : 3 * a.heads * kHead) / (32 * kNA)};
-  int longest = 0;
-  for (int x = 0; x < kOrderXcds; x++) longest = std::max(longest, order.length(x));
-  const dim3 grid(kOrderXcds * longest);
+  const ProjGrid g = proj_grid(out ? a.seq_len : a.seq_pad, out ? a.n_out : 3 * a.heads * kHead,
+                               32 * kMB, 32 * kNA);
+  a.tiles_m = g.order.tiles_m;
+  a.chunk = g.order.chunk;
+  const dim3 grid(kOrderXcds * g.longest);
   constexpr int kRef = H3HIP_ROUND_REFERENCE, kF32 = H3HIP_ROUND_FP32;
   if (out)
     proj_gemm_kernel<kNA, kMB, kRef, 8, true, true><<<grid, kThreads, 0, st>>>(a);
@@ -279,6 +284,8 @@ int launch_proj_gemm(const ProjArgs& a, ProjTile tile, int32_t rounding, bool pl
     case ProjTile::k256x192: return launch<8, 6>(a, rounding, plain, out, stream);
     case ProjTile::k256x160: return launch<8, 5>(a, rounding, plain, out, stream);
     case ProjTile::k256x128: return launch<8, 4>(a, rounding, plain, out, stream);
+    case ProjTile::k128x192: return launch<4, 6>(a, rounding, plain, out, stream);
+    case ProjTile::k128x160: return launch<4, 5>(a, rounding, plain, out, stream);
     case ProjTile::k128x128: return launch<4, 4>(a, rounding, plain, out, stream);
     default: return launch<4, 2>(a, rounding, plain, out, stream);
   }

@@ -15,6 +15,8 @@ enum class ProjTile {
   k256x192,
   k256x160,
   k256x128,
+  k128x192,
+  k128x160,
   k128x128,
   k128x64,
 };
@@ -26,25 +28,40 @@ struct ProjShape {
 };
 constexpr ProjShape kProjShapes[] = {
     {ProjTile::k256x256, 256, 256, 1.00}, {ProjTile::k256x224, 256, 224, 0.90},
-    {ProjTile::k256x192, 256, 192, 0.78}, {ProjTile::k256x160, 256, 160, 0.68},
-    {ProjTile::k256x128, 256, 128, 0.57}, {ProjTile::k128x128, 128, 128, 0.36},
-    {ProjTile::k128x64, 128, 64, 0.30},
+    {ProjTile::k256x192, 256, 192, 0.78}, {ProjTile::k256x160, 256, 160, 0.67},
+    {ProjTile::k256x128, 256, 128, 0.57}, {ProjTile::k128x192, 128, 192, 0.50},
+    {ProjTile::k128x160, 128, 160, 0.40}, {ProjTile::k128x128, 128, 128, 0.39},
+    {ProjTile::k128x64, 128, 64, 0.28},
 };
 
-// Tiles the longest XCD list gives each of its 32 CUs.
-inline int proj_rounds(int tokens, int channels, int tile_tokens, int tile_channels) {
-  const TileOrder order{(tokens + tile_tokens - 1) / tile_tokens, channels / tile_channels};
-  int longest = 0;
-  for (int x = 0; x < kOrderXcds; x++) longest = std::max(longest, order.length(x));
-  return (longest + 31) / 32;
+// The launch order of a grid, and how many tiles its longest XCD list gives
+// each of that XCD's 32 CUs. Chunks of four token tiles share the most in an
+// XCD's L2, but the lists then differ by up to two chunks, which can cost a
+// grid that just fits the chip a second round (252 tiles in lists of up to 34);
+// smaller chunks are taken when they save a round.
+struct ProjGrid {
+  TileOrder order;
+  int longest, rounds;
+};
+inline ProjGrid proj_grid(int tokens, int channels, int tile_tokens, int tile_channels) {
+  ProjGrid best{};
+  for (int chunk = kOrderChunk; chunk >= 1; chunk /= 2) {
+    ProjGrid g{{(tokens + tile_tokens - 1) / tile_tokens, channels / tile_channels, chunk}, 0, 0};
+    for (int x = 0; x < kOrderXcds; x++) g.longest = std::max(g.longest, g.order.length(x));
+    g.rounds = (g.longest + 31) / 32;
+    if (chunk == kOrderChunk || g.rounds < best.rounds) best = g;
+  }
+  return best;
 }
 
-// The tile whose rounds take the least time. A shape's cost is what MI355X
-// measures for it where all CUs are busy (0.88-0.92, 0.76-0.80, 0.66-0.70,
-// 0.56-0.60, 0.35-0.40 and 0.28-0.31 of a 256 x 256 tile over 22 token counts from 64 to
-// 18,102 and four layers); the picks were the fastest shape, or within 1.5% of
-// it, at 87 of those 88 sizes. Few tiles are where it matters: 2,048 tokens x
-// 5,120 channels are 160 tiles of 256 tokens (90 us) or 220 of 192 (80 us).
+// The tile whose rounds take the least time. A shape's cost is fitted to what
+// MI355X measures for it against a 256 x 256 tile's round (0.88-0.97, 0.76-0.93,
+// 0.63-0.84, 0.55-0.77, 0.42-0.57, 0.38-0.53, 0.33-0.47 and 0.23-0.35, from a full chip's
+// to an almost empty one's), over 64 sizes from 64 to 4,096 tokens of four layers:
+// the picks were the fastest shape or within 1.2% of it at 61 of them. Few
+// tiles are where it matters: 2,048 tokens x 5,120 channels are 160 tiles of 256
+// tokens (94 us) or 220 of 192 (87 us), 917 tokens 80 tiles (81 us), or 160 of 256 x
+// 128 (52 us) or 240 of 128 x 160 (42 us).
 //
 // With few reduction steps a tile is mostly its fill and epilogue: there the
 // eight-wave kernel, whose two waves per SIMD cover each other's epilogue, is
@@ -57,7 +74,7 @@ inline ProjTile pick_proj_tile(int tokens, int channels, int hidden, bool fused)
   double best = 0;
   ProjTile tile = ProjTile::kEightWave;
   for (const ProjShape& s : kProjShapes) {
-    const int rounds = proj_rounds(tokens, channels, s.tokens, s.channels);
+    const int rounds = proj_grid(tokens, channels, s.tokens, s.channels).rounds;
     const double cost = s.cost * rounds;
     if (s.tile == ProjTile::k256x256) {
       best = cost;

@@ -398,7 +398,7 @@ extern "C" int h3hip_qkv_proj(const void* x, int64_t ldx, const void* w, int64_t
              rope_table,
              static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(k_out),
              static_cast<uint16_t*>(v_out), ldx, ldw, eps, hidden, rot, seq_len, seq_pad, heads,
-             tiles_m, 0, 0};
+             tiles_m, 0, 0, 0};
   const ProjTile tile = pick_proj_tile(seq_pad, 3 * heads * kHD, hidden, !plain);
   if (tile != ProjTile::kEightWave)
     return launch_proj_gemm(a, tile, rounding, plain, false, as_stream(stream));
@@ -447,7 +447,7 @@ extern "C" int h3hip_out_proj(const void* x, int64_t ldx, const void* w, int64_t
              "tensors must be 16-byte aligned");
   ProjArgs a{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), nullptr, nullptr,
              nullptr, static_cast<uint16_t*>(y), nullptr, nullptr, ldx, ldw, 0.f, in_features,
-             128, seq_len, tiles_m * kPM, 1, tiles_m, out_features, ldy};
+             128, seq_len, tiles_m * kPM, 1, tiles_m, out_features, ldy, 0};
   const ProjTile tile = pick_proj_tile(seq_len, out_features, in_features, false);
   if (tile != ProjTile::kEightWave)
     return launch_proj_gemm(a, tile, H3HIP_ROUND_REFERENCE, true, true, as_stream(stream));

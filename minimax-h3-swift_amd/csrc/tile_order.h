@@ -10,12 +10,12 @@
 
 namespace h3hip {
 
-constexpr int kOrderChunk = 4;   // token tiles per chunk
+constexpr int kOrderChunk = 4;   // token tiles per chunk by default
 constexpr int kOrderXcds = 8;    // MI355X: 8 XCDs, workgroups dispatched round-robin
 
-// Launch order of the (token tile, channel tile) grid. A chunk is kOrderChunk
+// Launch order of the (token tile, channel tile) grid. A chunk is `chunk`
 // token tiles of one channel tile; chunk c = g * tiles_n + tn covers token
-// tiles kOrderChunk g .. (the last group may be short). Chunk c belongs to XCD
+// tiles chunk g .. (the last group may be short). Chunk c belongs to XCD
 // c % 8, which runs its chunks in order of c. So at any time the 8 XCDs work
 // on the same few token tiles, each on its own channel tiles: x is fetched
 // from HBM about once and shared through the last-level cache, W stays
@@ -25,28 +25,29 @@ constexpr int kOrderXcds = 8;    // MI355X: 8 XCDs, workgroups dispatched round-
 // flight than the 256 MB last-level cache holds at hidden 5120.
 struct TileOrder {
   int tiles_m, tiles_n;
+  int chunk = kOrderChunk;   // token tiles per chunk
   // Chunks c < n with c % 8 == x.
   __host__ __device__ int count(int n, int x) const { return n > x ? (n - 1 - x) / kOrderXcds + 1 : 0; }
-  __host__ __device__ int full_chunks() const { return (tiles_m / kOrderChunk) * tiles_n; }
-  __host__ __device__ int all_chunks() const { return ((tiles_m + kOrderChunk - 1) / kOrderChunk) * tiles_n; }
+  __host__ __device__ int full_chunks() const { return (tiles_m / chunk) * tiles_n; }
+  __host__ __device__ int all_chunks() const { return ((tiles_m + chunk - 1) / chunk) * tiles_n; }
   // Tiles XCD x runs.
   __host__ __device__ int length(int x) const {
     const int nf = full_chunks();
-    return kOrderChunk * count(nf, x) + (tiles_m % kOrderChunk) * (count(all_chunks(), x) - count(nf, x));
+    return chunk * count(nf, x) + (tiles_m % chunk) * (count(all_chunks(), x) - count(nf, x));
   }
   // The p-th tile (p < length(x)) XCD x runs, as token tile << 16 | channel tile.
   __host__ __device__ int tile(int x, int p) const {
     const int nf = full_chunks(), fx = count(nf, x);
     int c, i;
-    if (p < kOrderChunk * fx) {
-      c = x + kOrderXcds * (p / kOrderChunk);
-      i = p % kOrderChunk;
-    } else {   // the short chunks of the last group, tiles_m % kOrderChunk tiles each
-      const int r = tiles_m % kOrderChunk, q = p - kOrderChunk * fx;
+    if (p < chunk * fx) {
+      c = x + kOrderXcds * (p / chunk);
+      i = p % chunk;
+    } else {   // the short chunks of the last group, tiles_m % chunk tiles each
+      const int r = tiles_m % chunk, q = p - chunk * fx;
       c = nf + ((x - nf) % kOrderXcds + kOrderXcds) % kOrderXcds + kOrderXcds * (q / r);
       i = q % r;
     }
-    return (kOrderChunk * (c / tiles_n) + i) << 16 | (c % tiles_n);
+    return (chunk * (c / tiles_n) + i) << 16 | (c % tiles_n);
   }
 };
 

@@ -22,9 +22,11 @@ pytestmark = pytest.mark.gpu
     ("256x224", 801, 1024, 15360, None, None),
     ("256x192", 700, 1152, 15360, 1160, 15368),
     ("256x160", 600, 192, 15360, None, None),
-    ("256x128", 1001, 192, 5120, 200, 5128),
-    ("256x128", 1001, 64, 5120, None, None),
-    ("256x128", 897, 320, 5376, None, None),
+    ("256x128", 1201, 192, 5120, 200, 5128),
+    ("256x128", 1201, 64, 5120, None, None),
+    ("256x128", 1160, 320, 5376, None, None),
+    ("128x192", 1001, 192, 5120, None, None),
+    ("128x160", 900, 320, 5120, None, 5128),
     ("128x128", 400, 448, 5120, 456, None),
     ("128x64", 129, 64, 256, None, 264),
 ])
@@ -46,6 +48,8 @@ def test_out_proj(tile, S, fin, fout, ldx, ldy):
     ("256x160", 1100, 1536, 40, 128, 0),   # seq_pad 1,152 ends inside the eighth tile
     ("256x160", 600, 128, 40, 128, 1),
     ("256x128", 1250, 256, 14, 128, 0),
+    ("128x192", 300, 704, 40, 128, 1),
+    ("128x160", 800, 256, 14, 96, 0),      # seq_pad 896 ends inside the sixth tile
     ("128x128", 1000, 704, 6, 96, 0),
     ("128x64", 256, 64, 2, 96, 1),
 ] + [("128x64", 200, 64 * k, 2, 128, 0) for k in range(2, 8)])
