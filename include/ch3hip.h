@@ -138,7 +138,8 @@ int h3hip_plan_tiles(h3hip_plan plan, int32_t* row_ptr, int32_t* col_idx);
 double h3hip_plan_density(h3hip_plan plan);
 
 /* The attention launch's persistent schedule for a plan with these CSR rows
- * (host-side, synchronous; h3hip_plan_create builds the same lists). No
+ * (host-side, synchronous; h3hip_plan_create builds the same lists, or lists of
+ * half units of 64 queries where few or uneven units make that end earlier). No
  * counterpart in the reference, whose MLX dispatch has no persistent
  * workgroups; exposed so callers and tests can inspect which (head, q-tile)
  * units each workgroup runs. row_ptr[n_tiles + 1]; groups = workgroups, a

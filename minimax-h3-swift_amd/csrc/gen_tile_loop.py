@@ -47,6 +47,8 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 OUT = os.path.join(HERE, "bsattn_tile_loop.inc")
+SOURCE = "gen_tile_loop.py"
+MACRO = "H3_TILE_LOOP"
 
 WAVES = 8                      # per workgroup, two per SIMD
 ROWS_PER_WAVE = 128 // WAVES   # rows of each K/V tile one wave loads
@@ -297,16 +299,17 @@ def rsrc_setup(which, col, base_lo, base_hi, rec, stride128):
 
 def dma_lines(which, slot):
     """This wave's buffer loads of its rows of a K or V tile into the slot,
-    in order: one M0 for the tile, the loads' instruction offsets (which
-    apply to the LDS and to the global address alike) for their 1 KiB steps;
-    the lane offsets v[DK0/DV0 + i] are lowered by the same 1024 i."""
+    in order: one M0 for (up to) four loads, their instruction offsets (which
+    apply to the LDS and to the global address alike) for the 1 KiB steps;
+    the lane offsets v[DK0/DV0 + i] are lowered by the same 1024 (i & 3)."""
     m0 = "%[m0k]" if which == "k" else "%[m0v]"
     base = DK0 if which == "k" else DV0
     rs = KRS if which == "k" else VRS
     out = []
     for i in range(LOADS):
-        ld = f"buffer_load_dwordx4 v{base + i}, {rs}, 0 offen offset:{1024 * i} lds"
-        out.append(([f"s_add_u32 m0, {m0}, {slot * KSLOT}", "s_nop 0"] if i == 0 else []) + [ld])
+        ld = f"buffer_load_dwordx4 v{base + i}, {rs}, 0 offen offset:{1024 * (i & 3)} lds"
+        pre = [f"s_add_u32 m0, {m0}, {slot * KSLOT + 1024 * i}", "s_nop 0"] if i % 4 == 0 else []
+        out.append(pre + [ld])
     return out
 
 
@@ -599,12 +602,12 @@ def render() -> str:
     cl = ", ".join(f'"{r}"' for r in clobbers())
     n_mfma = sum(1 for ln in lines if ln.startswith("v_mfma"))
     return (
-        "// Generated by gen_tile_loop.py -- do not edit; regenerate instead.\n"
+        f"// Generated by {SOURCE} -- do not edit; regenerate instead.\n"
         f"// {len(lines)} lines, {n_mfma} MFMAs.\n"
-        f"#define H3_TILE_LOOP_WAVES {WAVES}\n"
-        f"#define H3_TILE_LOOP_ROWS_PER_WAVE {ROWS_PER_WAVE}\n"
-        "#define H3_TILE_LOOP_ASM \\\n" + body.replace("\n", " \\\n") + "\n\n"
-        "#define H3_TILE_LOOP_CLOBBERS " + cl + "\n")
+        f"#define {MACRO}_WAVES {WAVES}\n"
+        f"#define {MACRO}_ROWS_PER_WAVE {ROWS_PER_WAVE}\n"
+        f"#define {MACRO}_ASM \\\n" + body.replace("\n", " \\\n") + "\n\n"
+        f"#define {MACRO}_CLOBBERS " + cl + "\n")
 
 
 def main() -> int:

@@ -22,6 +22,7 @@ struct h3hip_plan_s {
   // b % 8) runs the units work[work_ptr[b] .. work_ptr[b + 1]), each
   // (head << 16 | q_tile), in order.
   int32_t groups = 0;
+  bool half_units = false;        // units of 64 queries: work holds head << 16 | half row
   std::vector<int32_t> work_ptr;  // [groups + 1]
   std::vector<int32_t> work;
   int32_t* d_row_ptr = nullptr;
@@ -40,7 +41,8 @@ constexpr size_t kListAlign = 64;  // int32 entries
 
 // Unit descriptor layout: unit (head << 16 | q_tile), first index of the row
 // in col_idx, tile count n, columns c0, c1, c2 (the first three, repeating the
-// last when n < 3), ragged (1 when the last tile runs past seq_len), unused.
+// last when n < 3), ragged (1 when the last tile runs past seq_len), first query
+// row within the q-tile (0, or 64 for the second of two half units).
 constexpr int kUnitDescInts = 8;
 
 namespace h3hip {

@@ -1,6 +1,7 @@
 // The attention kernel's persistent schedule, built on the host from a plan's
-// row lengths. Pure C++, no device code: h3hip_plan_create uploads the result,
-// and h3hip_schedule exposes the same lists to callers and tests.
+// row lengths. Pure C++, no device code: h3hip_plan_create uploads the result
+// (over half rows where those end earlier, tile_plan.hip), and h3hip_schedule
+// exposes the lists over whole rows to callers and tests.
 #include <algorithm>
 #include <cstdint>
 #include <numeric>

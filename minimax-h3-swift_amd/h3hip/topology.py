@@ -118,7 +118,8 @@ def schedule(row_ptr: np.ndarray, heads: int, groups: int = 256):
     """The attention launch's persistent schedule for these CSR rows
     (h3hip_schedule): (work_ptr [groups + 1], work [heads * n_tiles]) int32;
     workgroup b runs work[work_ptr[b]:work_ptr[b + 1]], each unit
-    head << 16 | q_tile. The same lists h3hip_plan_create uploads."""
+    head << 16 | q_tile. h3hip_plan_create uploads the same lists, or a list of half
+    units (64 queries) where few or uneven units make that end earlier."""
     rp = np.ascontiguousarray(row_ptr, dtype=np.int32)
     n = len(rp) - 1
     work_ptr = np.zeros(groups + 1, dtype=np.int32)
