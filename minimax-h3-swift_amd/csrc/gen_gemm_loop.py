@@ -241,7 +241,6 @@ def render():
         acc = [f'"=&{{a[{32 * i}:{32 * i + 31}]}}"(C[{i}])' for i in range(-(-na * mb // 8))]
         out += [f"// {32 * na} channels x {32 * mb} tokens: {len(lines)} lines.",
                 f"#define H3_GEMM_LDS_{name} {g.lds}",
-                f"#define H3_GEMM_X_AT_{name} {g.x_at}",
                 f"#define H3_GEMM_BASES_{name} {g.bases}",
                 f"#define H3_GEMM_LOOP_{name} \\\n" + body + "\n",
                 f"#define H3_GEMM_OUT_{name}(C) " + ", ".join(acc),

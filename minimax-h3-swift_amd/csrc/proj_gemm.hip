@@ -62,8 +62,7 @@ struct Shape;
 #define H3_SHAPE(NA, MB, NAME)                                                               \
   template <>                                                                                \
   struct Shape<NA, MB> {                                                                     \
-    static constexpr int kLds = H3_GEMM_LDS_##NAME, kXAt = H3_GEMM_X_AT_##NAME,              \
-                         kBases = H3_GEMM_BASES_##NAME;                                      \
+    static constexpr int kLds = H3_GEMM_LDS_##NAME, kBases = H3_GEMM_BASES_##NAME;                   \
     static __device__ __forceinline__ void reduce(f32x32 (&c)[kAccs<NA, MB>], const int* ra,   \
                                                   const int* rb, const int* xv, const int* wv, \
                                                   uint32_t x_lo, uint32_t x_hi, uint32_t x_rec, \
