@@ -46,9 +46,10 @@ constexpr int kMaskCols = 256;
 
 // Bitmap of the rule over tile pairs (mask_rule.h): workgroup (x, y) answers
 // query tile y and key tiles 256x .. + 255. What bounds it is the launch and the
-// chain of integer divisions that places a tile in the lattice: 8.6 us at 250 x
-// 250 tiles of the local rule on MI355X, where testing the token pairs, six
-// divisions each, took 1,111 us.
+// chain of integer divisions that places a tile in the lattice. On MI355X, 250 x
+// 250 tiles of the local rule take 4.2 us in 24 x 42 frames (testing the token
+// pairs, six divisions each: 1,111 us), and with frames of any size a call among
+// others stays below 10 us, one-token rows included.
 __global__ __launch_bounds__(kMaskCols) void mask_rule_kernel(RuleDev r, uint8_t* bitmap) {
   const int32_t qi = blockIdx.y, kj = blockIdx.x * kMaskCols + threadIdx.x;
   const bool in_range = kj < r.n_tiles;
@@ -58,20 +59,13 @@ __global__ __launch_bounds__(kMaskCols) void mask_rule_kernel(RuleDev r, uint8_t
       *dst = r.kind == H3HIP_RULE_DENSE || abs(qi - kj) <= r.band || r.col_global[kj] ? 1 : 0;
     return;
   }
-  __shared__ RowSegment seg[kMaxSegs];
+  if (!in_range) return;
   const bool q_prefix = tile_in_prefix(r, qi);
   const TileSpan q = tile_span(r, qi);
-  const int32_t n_seg = q_prefix || r.kind != H3HIP_RULE_LOCAL ? 0 : q.row1 - q.row0 + 1;
-  if ((int)threadIdx.x < n_seg) {
-    const int32_t row = q.row0 + threadIdx.x, f = row / r.height;
-    seg[threadIdx.x] = row_segment(r, q, row, f, row - f * r.height);
-  }
-  __syncthreads();
-  if (!in_range) return;
-  *dst = q_prefix || tile_in_prefix(r, kj) ||
-                 lattice_tiles_see(r, q, tile_span(r, kj), seg, n_seg)
-             ? 1
-             : 0;
+  RuleBox box[kMaxBoxes] = {};
+  if (!q_prefix && r.kind == H3HIP_RULE_LOCAL) tile_boxes(r, q, box);
+  *dst = q_prefix || tile_in_prefix(r, kj) || lattice_tiles_see(r, q, tile_span(r, kj), box) ? 1
+                                                                                          : 0;
 }
 
 static dim3 mask_grid(int32_t n_tiles) {

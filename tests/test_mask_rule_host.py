@@ -18,19 +18,27 @@ CSRC = os.path.join(ROOT, "minimax-h3-swift_amd", "csrc")
 HARNESS = r"""
 #include "mask_rule.h"
 using namespace h3hip;
+// Calls of the header's functions (g++ -finstrument-functions).
+static long calls = 0;
+extern "C" {
+__attribute__((no_instrument_function)) void __cyg_profile_func_enter(void*, void*) { calls++; }
+__attribute__((no_instrument_function)) void __cyg_profile_func_exit(void*, void*) {}
+__attribute__((no_instrument_function)) long take_calls() {
+  const long c = calls;
+  calls = 0;
+  return c;
+}
+}
 extern "C" void bitmap(const int32_t* p, const uint8_t* landmark, uint8_t* out) {
   const RuleDev r{p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], 0, p[10], nullptr,
                   landmark};
   for (int32_t q = 0; q < r.n_tiles; q++) {
-    RowSegment seg[kMaxSegs];
-    int32_t n_seg = 0;
+    RuleBox box[kMaxBoxes] = {};
     const TileSpan s = tile_span(r, q);
-    if (r.kind == H3HIP_RULE_LOCAL && !tile_in_prefix(r, q))
-      for (int32_t row = s.row0; row <= s.row1; row++)
-        seg[n_seg++] = row_segment(r, s, row, row / r.height, row % r.height);
+    if (r.kind == H3HIP_RULE_LOCAL && !tile_in_prefix(r, q)) tile_boxes(r, s, box);
     for (int32_t k = 0; k < r.n_tiles; k++)
       out[q * r.n_tiles + k] = tile_in_prefix(r, q) || tile_in_prefix(r, k) ||
-                               lattice_tiles_see(r, s, tile_span(r, k), seg, n_seg);
+                               lattice_tiles_see(r, s, tile_span(r, k), box);
   }
 }
 """
@@ -74,9 +82,24 @@ def rules(tmp_path_factory):
     d = tmp_path_factory.mktemp("mask_rule")
     src, so = d / "h.cpp", d / "h.so"
     src.write_text(HARNESS)
-    subprocess.run([cxx, "-O1", "-std=c++17", "-fPIC", "-shared", "-I", CSRC, str(src), "-o",
+    subprocess.run([cxx, "-O1", "-std=c++17", "-fPIC", "-shared", "-finstrument-functions",
+                    "-Wl,-Bsymbolic", "-I", CSRC, str(src), "-o",
                     str(so)], check=True)
-    return ctypes.CDLL(str(so))
+    lib = ctypes.CDLL(str(so))
+    lib.take_calls.restype = ctypes.c_long
+    return lib
+
+
+def _bitmap(rules, rule, f, sp, fw, sw, lm):
+    flags = np.zeros(f, np.uint8)
+    flags[list(lm)] = 1
+    p = np.array([rule.kind, rule.seq_len, rule.prefix_len, f, rule.height, rule.width, fw, sp[0],
+                  sp[1], sw, rule.n_tiles], np.int32)
+    got = np.zeros((rule.n_tiles, rule.n_tiles), np.uint8)
+    u8 = ctypes.POINTER(ctypes.c_uint8)
+    rules.bitmap(p.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)),
+                 flags.ctypes.data_as(u8) if lm else None, got.ctypes.data_as(u8))
+    return got
 
 
 @pytest.mark.parametrize("case", CASES + _drawn(40))
@@ -85,11 +108,20 @@ def test_tile_pairs_match_token_pairs(rules, orc, case):
     seq = prefix + f * h * w
     rule = orc.Rule(kind, seq, prefix_len=prefix, frames=f, height=h, width=w, frame_window=fw,
                     sp_tile=sp, sp_window=sw, landmarks=list(lm))
-    flags = np.zeros(f, np.uint8)
-    flags[list(lm)] = 1
-    p = np.array([kind, seq, prefix, f, h, w, fw, sp[0], sp[1], sw, rule.n_tiles], np.int32)
-    got = np.zeros((rule.n_tiles, rule.n_tiles), np.uint8)
-    u8 = ctypes.POINTER(ctypes.c_uint8)
-    rules.bitmap(p.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)),
-                 flags.ctypes.data_as(u8) if lm else None, got.ctypes.data_as(u8))
+    got = _bitmap(rules, rule, f, sp, fw, sw, lm)
     assert np.array_equal(got, orc.tile_bitmap(rule))
+
+
+@pytest.mark.parametrize("f,h,w", [(2048, 1, 1), (1, 2048, 1), (16, 128, 1), (256, 2, 4),
+                                   (128, 4, 4), (32, 8, 8), (2, 32, 32)])
+def test_a_tile_pair_costs_the_same_however_narrow_the_lattice(rules, orc, f, h, w):
+    """LOCAL with windows that see only the token itself, so that nothing ends
+    the comparison early: 5 x 5 boxes of three axes each. (Row by row, a
+    pair of tiles of one-token rows is 16,384 comparisons.)"""
+    rule = orc.Rule(LOCAL, f * h * w, frames=f, height=h, width=w, frame_window=0,
+                    sp_tile=(1, 1), sp_window=0)
+    rules.take_calls()
+    got = _bitmap(rules, rule, f, (1, 1), 0, 0, ())
+    calls = rules.take_calls()
+    assert np.array_equal(got, orc.tile_bitmap(rule))
+    assert 0 < calls <= (25 * 5 + 64) * got.size, calls / got.size
