@@ -35,6 +35,12 @@ struct TileOrder {
     const int nf = full_chunks();
     return chunk * count(nf, x) + (tiles_m % chunk) * (count(all_chunks(), x) - count(nf, x));
   }
+  // Tiles the longest list holds: within the XCDs that run one full chunk more
+  // than the others, and within the others, the first runs the most.
+  __host__ __device__ int longest() const {
+    const int first = length(0), rest = length(full_chunks() % kOrderXcds);
+    return first > rest ? first : rest;
+  }
   // The p-th tile (p < length(x)) XCD x runs, as token tile << 16 | channel tile.
   __host__ __device__ int tile(int x, int p) const {
     const int nf = full_chunks(), fx = count(nf, x);
