@@ -208,8 +208,8 @@ __global__ __launch_bounds__(kThreads, 1) void proj_gemm_kernel(ProjArgs a) {
   const TileOrder order{a.tiles_m, n_total / kChannels, a.chunk};
   const int xcd = blockIdx.x % kOrderXcds, slot = blockIdx.x / kOrderXcds;
   if (slot >= order.length(xcd)) return;
-  const int tile = order.tile(xcd, slot);
-  const int m0 = (tile >> 16) * kTokens, n0 = (tile & 0xffff) * kChannels;
+  const uint32_t tile = order.tile(xcd, slot);
+  const int m0 = (int)(tile >> 16) * kTokens, n0 = (int)(tile & 0xffff) * kChannels;
 
   const int lr = lane & 15, g = lane >> 4;
   const uint32_t lds_base = uniform((uint32_t)(size_t)(__attribute__((address_space(3))) uint16_t*)lds);

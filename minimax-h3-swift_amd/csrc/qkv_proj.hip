@@ -128,8 +128,8 @@ __global__ __launch_bounds__(kPThreads, 1) void qkv_proj_kernel(ProjArgs a) {
   const TileOrder order{a.tiles_m, tiles_n};
   const int xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
   if (slot >= order.length(xcd)) return;
-  const int tile = order.tile(xcd, slot);
-  const int m0 = (tile >> 16) * kPM, n0 = (tile & 0xffff) * kPN;
+  const uint32_t tile = order.tile(xcd, slot);
+  const int m0 = (int)(tile >> 16) * kPM, n0 = (int)(tile & 0xffff) * kPN;
   const int part = kOut ? 0 : n0 / inner;                   // uniform over the tile
   const int head = kOut ? 0 : (n0 - part * inner) / kHD + nh;   // this wave's head
 

@@ -3,6 +3,8 @@
 // covers every tile exactly once.
 #pragma once
 
+#include <cstdint>
+
 #ifndef __HIPCC__
 #define __host__
 #define __device__
@@ -41,8 +43,9 @@ struct TileOrder {
     const int first = length(0), rest = length(full_chunks() % kOrderXcds);
     return first > rest ? first : rest;
   }
-  // The p-th tile (p < length(x)) XCD x runs, as token tile << 16 | channel tile.
-  __host__ __device__ int tile(int x, int p) const {
+  // The p-th tile (p < length(x)) XCD x runs, as token tile << 16 | channel tile:
+  // unsigned, for x and W of up to 2 GiB have up to 65,535 tiles of 256 rows.
+  __host__ __device__ uint32_t tile(int x, int p) const {
     const int nf = full_chunks(), fx = count(nf, x);
     int c, i;
     if (p < chunk * fx) {
@@ -53,7 +56,7 @@ struct TileOrder {
       c = nf + ((x - nf) % kOrderXcds + kOrderXcds) % kOrderXcds + kOrderXcds * (q / r);
       i = q % r;
     }
-    return (chunk * (c / tiles_n) + i) << 16 | (c % tiles_n);
+    return (uint32_t)(chunk * (c / tiles_n) + i) << 16 | (uint32_t)(c % tiles_n);
   }
 };
 

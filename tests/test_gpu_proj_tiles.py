@@ -74,3 +74,21 @@ def test_padding_rows_past_the_last_token_tile():
         torch.cuda.synchronize()
         _check_plain(*out, x, w, S)
         assert all((bits(t[:, S:]) == 0).all() for t in out)
+
+
+def test_more_token_tiles_than_a_signed_half_word():
+    """32,770 token tiles of 256: rows on both sides of tile 32,768 and the last
+    (a 1 GiB x; its one-step product keeps the run short)."""
+    from h3hip import ops
+    S, fin, fout = 32769 * 256 + 3, 64, 256
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    x = torch.empty((S, fin), dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    w = torch.randn((fout, fin), generator=g, device="cuda").to(torch.bfloat16)
+    note(f"out_proj S={S} in={fin} out={fout}")
+    y = ops.out_proj(x, w)
+    torch.cuda.synchronize()
+    edge = 32768 * 256
+    for r in (0, 1000, edge - 256, edge, edge + 255, S - 3):
+        rows = slice(r, min(S, r + 256))
+        _check_fp32(y[rows], x[rows], w)

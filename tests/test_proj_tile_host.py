@@ -51,13 +51,14 @@ int main(int argc, char** argv) {
     for (int a = 2; a + 3 < argc; a += 4) {
       const h3hip::ProjGrid g = h3hip::proj_grid(std::atoi(argv[a]), std::atoi(argv[a + 1]),
                                                  std::atoi(argv[a + 2]), std::atoi(argv[a + 3]));
-      std::set<int> seen;
+      std::set<long> seen;
       int n = 0, longest = 0;
       for (int x = 0; x < h3hip::kOrderXcds; x++) {
         longest = std::max(longest, g.order.length(x));
         for (int p = 0; p < g.order.length(x); p++, n++) {
-          const int t = g.order.tile(x, p);
-          if ((t >> 16) < g.order.tiles_m && (t & 0xffff) < g.order.tiles_n) seen.insert(t);
+          const auto t = g.order.tile(x, p);
+          const int tm = (int)(t >> 16), tn = (int)(t & 0xffff);   // as the kernels read it
+          if (tm >= 0 && tm < g.order.tiles_m && tn < g.order.tiles_n) seen.insert(t);
         }
       }
       std::printf("%d %d %d\n", n == g.order.tiles_m * g.order.tiles_n && n == (int)seen.size() &&
@@ -130,7 +131,8 @@ def test_launch_orders_list_every_tile_once(pick):
     fewest rounds, 252 tiles in one; every tile once in each order."""
     cases = [(896, 5376, 160, 128), (31885, 15360, 256, 256), (1, 256, 64, 128),
              (1152, 21504, 192, 256), (917, 5120, 160, 128), (300, 5120, 64, 128),
-             (641, 15360, 160, 256), (2048, 5120, 192, 256), (18102, 5376, 224, 256)]
+             (641, 15360, 160, 256), (2048, 5120, 192, 256), (18102, 5376, 224, 256),
+             (8388609, 256, 256, 256), (16776960, 256, 256, 256), (256, 16776960, 256, 256)]
     got = pick.grids(cases)
     assert all(ok for ok, _, _ in got), got
     assert got[0][2] == 1 and got[0][1] < 4
