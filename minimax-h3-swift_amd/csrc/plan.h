@@ -57,4 +57,9 @@ void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 int build_schedule(const std::vector<int32_t>& row_ptr, int32_t heads, int32_t groups,
                    std::vector<int32_t>& work_ptr, std::vector<int32_t>& work);
 
+// The schedule of a plan with these CSR rows: build_schedule's, or with half_units
+// set lists of half units, (head << 16 | 2 q_tile + half) listed once each.
+int plan_schedule(const std::vector<int32_t>& row_ptr, int32_t heads, int32_t groups,
+                  bool& half_units, std::vector<int32_t>& work_ptr, std::vector<int32_t>& work);
+
 }  // namespace h3hip

@@ -1,11 +1,13 @@
 // The attention kernel's persistent schedule, built on the host from a plan's
-// row lengths. Pure C++, no device code: h3hip_plan_create uploads the result
-// (over half rows where those end earlier, tile_plan.hip), and h3hip_schedule
-// exposes the lists over whole rows to callers and tests.
+// row lengths. Pure C++, no device code, so CPU tests can compile it:
+// h3hip_plan_create uploads plan_schedule's lists (over half rows where those end
+// earlier) and h3hip_plan_schedule gives them back; h3hip_schedule exposes the
+// lists over whole rows.
 #include <algorithm>
 #include <cstdint>
 #include <numeric>
 #include <queue>
+#include <utility>
 #include <vector>
 
 #include "plan.h"
@@ -69,6 +71,24 @@ static void deal(const std::vector<int32_t>& list, const std::vector<int32_t>& l
     free_at[then] |= c;
     wg.push_back(__builtin_ctzll(c));
   }
+}
+
+// Every (head, row) unit exactly once: a dropped unit would leave its output rows
+// unwritten, a duplicated one would race with itself.
+static int check_units(int32_t heads, int32_t rows, const std::vector<int32_t>& work) {
+  std::vector<uint8_t> seen((size_t)heads * rows, 0);
+  bool ok = work.size() == (size_t)heads * rows;
+  for (size_t i = 0; ok && i < work.size(); i++) {
+    const int32_t h = work[i] >> 16, r = work[i] & 0xffff;
+    ok = h >= 0 && h < heads && r < rows && !seen[(size_t)h * rows + r];
+    if (ok) seen[(size_t)h * rows + r] = 1;
+  }
+  if (!ok) {
+    set_error("internal: the attention schedule does not list each of the %lld units once",
+              (long long)heads * rows);
+    return H3HIP_EHIP;
+  }
+  return H3HIP_OK;
 }
 
 int build_schedule(const std::vector<int32_t>& row_ptr, int32_t heads, int32_t groups,
@@ -149,23 +169,82 @@ int build_schedule(const std::vector<int32_t>& row_ptr, int32_t heads, int32_t g
   size_t at = 0;
   for (int x = 0; x < kXcd; x++)
     for (int32_t u : lists[x]) work[next[wg[at++]]++] = u;
-  // Every (head, q-tile) unit exactly once: a dropped unit would leave its
-  // output rows unwritten, a duplicated one would race with itself.
-  std::vector<uint8_t> seen((size_t)heads * nq, 0);
-  bool ok = work.size() == (size_t)heads * nq;
-  for (size_t i = 0; ok && i < work.size(); i++) {
-    const int32_t h = work[i] >> 16, qt = work[i] & 0xffff;
-    ok = h >= 0 && h < heads && qt < nq && !seen[(size_t)h * nq + qt];
-    if (ok) seen[(size_t)h * nq + qt] = 1;
+  return check_units(heads, nq, work);
+}
+
+// One unit per workgroup at most (heads x rows <= groups), a contiguous range per
+// XCD, so that the units of a head share its L2.
+static int spread_units(int32_t heads, int32_t rows, int32_t groups,
+                        std::vector<int32_t>& work_ptr, std::vector<int32_t>& work) {
+  const int64_t units = (int64_t)heads * rows;
+  std::vector<int32_t> at(groups, -1);
+  for (int x = 0; x < 8; x++) {
+    const int32_t first = (int32_t)(units * x / 8), last = (int32_t)(units * (x + 1) / 8);
+    for (int32_t i = first; i < last; i++) at[(i - first) * 8 + x] = (i / rows) << 16 | i % rows;
   }
-  if (!ok) {
-    set_error("internal: the attention schedule does not list each of the %lld units once",
-              (long long)heads * nq);
-    return H3HIP_EHIP;
+  work.clear();
+  work_ptr.assign(groups + 1, 0);
+  for (int32_t b = 0; b < groups; b++) {
+    if (at[b] >= 0) work.push_back(at[b]);
+    work_ptr[b + 1] = (int32_t)work.size();
+  }
+  return check_units(heads, rows, work);
+}
+
+// Cost of a unit beyond its tiles and of a tile, in full units' tiles, where a
+// workgroup runs few units: dense rows of 8, 17 and 42 tiles, one unit each, take
+// 15.4, 25.1 and 52.2 us in full units and 11.3, 18.9 and 42.2 in half ones on MI355X,
+// launch included.
+constexpr double kFullUnit = 2.0, kHalfUnit = 1.7, kHalfTile = 0.85;
+// Full units per workgroup up to which half units are looked at. Past it a
+// launch is bound by the chip's throughput, where half units cost 1.2-1.3 times.
+constexpr int kHalfUnitsUpTo = 6;
+
+// The time the cost model gives the longest workgroup of these lists.
+static double longest_workgroup(const std::vector<int32_t>& row_ptr,
+                                const std::vector<int32_t>& work_ptr,
+                                const std::vector<int32_t>& work, double unit, double tile) {
+  double worst = 0;
+  for (size_t b = 0; b + 1 < work_ptr.size(); b++) {
+    double t = 0;
+    for (int32_t i = work_ptr[b]; i < work_ptr[b + 1]; i++) {
+      const int32_t row = work[i] & 0xffff;
+      t += unit + tile * (row_ptr[row + 1] - row_ptr[row]);
+    }
+    worst = std::max(worst, t);
+  }
+  return worst;
+}
+
+// Whole units, or half units (64 queries, bsattn_half.hip) where their longest
+// workgroup ends earlier: few units (917 tokens x 8 heads: 15.9 -> 11.8 us), or few
+// long rows among short ones (31,885 tokens x 2 heads of the local rule, whose 5
+// prefix rows see all 250 tiles: 295 -> 236 us).
+int plan_schedule(const std::vector<int32_t>& row_ptr, int32_t heads, int32_t groups,
+                  bool& half_units, std::vector<int32_t>& work_ptr, std::vector<int32_t>& work) {
+  half_units = false;
+  int rc = build_schedule(row_ptr, heads, groups, work_ptr, work);
+  if (rc != H3HIP_OK) return rc;
+  const int32_t n = (int32_t)row_ptr.size() - 1;
+  if ((int64_t)heads * n > kHalfUnitsUpTo * (int64_t)groups) return H3HIP_OK;
+  std::vector<int32_t> half_rows(2 * (size_t)n + 1, 0), half_ptr, half_work;
+  for (size_t r = 0; r + 1 < half_rows.size(); r++)
+    half_rows[r + 1] = half_rows[r] + row_ptr[r / 2 + 1] - row_ptr[r / 2];
+  // build_schedule balances the XCDs by cost and gives some workgroups two units
+  // where each could have one (4,096 tokens x 4 heads of a band: 15.4 us, spread
+  // 11.1, full units 14.1).
+  rc = 2 * (int64_t)heads * n <= groups
+           ? spread_units(heads, 2 * n, groups, half_ptr, half_work)
+           : build_schedule(half_rows, heads, groups, half_ptr, half_work);
+  if (rc != H3HIP_OK) return rc;
+  if (longest_workgroup(half_rows, half_ptr, half_work, kHalfUnit, kHalfTile) <
+      longest_workgroup(row_ptr, work_ptr, work, kFullUnit, 1.0)) {
+    half_units = true;
+    work_ptr = std::move(half_ptr);
+    work = std::move(half_work);
   }
   return H3HIP_OK;
 }
-
 
 }  // namespace h3hip
 

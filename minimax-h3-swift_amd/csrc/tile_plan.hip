@@ -333,71 +333,6 @@ static int launch_row_ptr(const uint8_t* d_bitmap, int32_t nq, int32_t nk, int32
   return check_launch("scan_kernel");
 }
 
-// One unit per workgroup at most (heads x rows <= groups), a contiguous range per
-// XCD, so that the units of a head share its L2.
-static void spread_units(int32_t heads, int32_t rows, int32_t groups,
-                         std::vector<int32_t>& work_ptr, std::vector<int32_t>& work) {
-  const int64_t units = (int64_t)heads * rows;
-  std::vector<int32_t> at(groups, -1);
-  for (int x = 0; x < 8; x++) {
-    const int32_t first = (int32_t)(units * x / 8), last = (int32_t)(units * (x + 1) / 8);
-    for (int32_t i = first; i < last; i++) at[(i - first) * 8 + x] = (i / rows) << 16 | i % rows;
-  }
-  work.clear();
-  work_ptr.assign(groups + 1, 0);
-  for (int32_t b = 0; b < groups; b++) {
-    if (at[b] >= 0) work.push_back(at[b]);
-    work_ptr[b + 1] = (int32_t)work.size();
-  }
-}
-
-// Cost of a unit beyond its tiles and of a tile, in full units' tiles, where a
-// workgroup runs few units: dense rows of 8, 17 and 42 tiles, one unit each, take
-// 15.4, 25.1 and 52.2 us in full units and 11.3, 18.9 and 42.2 in half ones on MI355X,
-// launch included.
-constexpr double kFullUnit = 2.0, kHalfUnit = 1.7, kHalfTile = 0.85;
-// Full units per workgroup up to which half units are looked at. Past it a
-// launch is bound by the chip's throughput, where half units cost 1.2-1.3 times.
-constexpr int kHalfUnitsUpTo = 6;
-
-// Replaces the plan's schedule by one of half units (64 queries, bsattn_half.hip)
-// where its longest workgroup ends earlier: few units (917 tokens x 8 heads: 15.9
-// -> 11.8 us), or few long rows among short ones (31,885 tokens x 2 heads of the
-// local rule, whose 5 prefix rows see all 250 tiles: 295 -> 236 us).
-static int try_half_units(h3hip_plan p) {
-  if ((int64_t)p->heads * p->n_tiles > kHalfUnitsUpTo * (int64_t)p->groups) return H3HIP_OK;
-  std::vector<int32_t> rows(2 * (size_t)p->n_tiles + 1, 0), work_ptr, work;
-  for (size_t r = 0; r + 1 < rows.size(); r++)
-    rows[r + 1] = rows[r] + p->row_ptr[r / 2 + 1] - p->row_ptr[r / 2];
-  // build_schedule balances the XCDs by cost and gives some workgroups two units
-  // where each could have one (4,096 tokens x 4 heads of a band: 15.4 us, spread
-  // 11.1, full units 14.1).
-  if (2 * (int64_t)p->heads * p->n_tiles <= p->groups) {
-    spread_units(p->heads, 2 * p->n_tiles, p->groups, work_ptr, work);
-  } else {
-    const int rc = build_schedule(rows, p->heads, p->groups, work_ptr, work);
-    if (rc != H3HIP_OK) return rc;
-  }
-  auto longest = [&](const std::vector<int32_t>& wp, const std::vector<int32_t>& w,
-                     const std::vector<int32_t>& rp, double unit, double tile) {
-    double worst = 0;
-    for (int32_t b = 0; b < p->groups; b++) {
-      double t = 0;
-      for (int32_t i = wp[b]; i < wp[b + 1]; i++)
-        t += unit + tile * (rp[(w[i] & 0xffff) + 1] - rp[w[i] & 0xffff]);
-      worst = std::max(worst, t);
-    }
-    return worst;
-  };
-  if (longest(work_ptr, work, rows, kHalfUnit, kHalfTile) <
-      longest(p->work_ptr, p->work, p->row_ptr, kFullUnit, 1.0)) {
-    p->half_units = true;
-    p->work_ptr = std::move(work_ptr);
-    p->work = std::move(work);
-  }
-  return H3HIP_OK;
-}
-
 }  // namespace h3hip
 
 using namespace h3hip;
@@ -580,9 +515,7 @@ int h3hip_plan_create(const h3hip_mask_rule* rule, int32_t heads, const h3hip_po
     return fail(H3HIP_EHIP);
   }
   p->groups = std::max(8, cus / 8 * 8);
-  rc = build_schedule(p->row_ptr, heads, p->groups, p->work_ptr, p->work);
-  if (rc) return fail(rc);
-  rc = try_half_units(p);
+  rc = plan_schedule(p->row_ptr, heads, p->groups, p->half_units, p->work_ptr, p->work);
   if (rc) return fail(rc);
   const size_t units = p->work.size();
   auto aligned = [](size_t ints) { return (ints + kListAlign - 1) / kListAlign * kListAlign; };
@@ -644,6 +577,16 @@ int h3hip_plan_tiles(h3hip_plan p, int32_t* row_ptr, int32_t* col_idx) {
   H3_REQUIRE(p != nullptr, H3HIP_EINVAL, "plan is NULL");
   if (row_ptr) std::memcpy(row_ptr, p->row_ptr.data(), sizeof(int32_t) * p->row_ptr.size());
   if (col_idx && p->nnz > 0) std::memcpy(col_idx, p->col_idx.data(), sizeof(int32_t) * p->nnz);
+  return H3HIP_OK;
+}
+
+int h3hip_plan_schedule(h3hip_plan p, int32_t* unit_rows, int32_t* groups, int32_t* work_ptr,
+                        int32_t* work) {
+  H3_REQUIRE(p != nullptr, H3HIP_EINVAL, "plan is NULL");
+  if (unit_rows) *unit_rows = p->half_units ? H3HIP_TILE / 2 : H3HIP_TILE;
+  if (groups) *groups = p->groups;
+  if (work_ptr) std::copy(p->work_ptr.begin(), p->work_ptr.end(), work_ptr);
+  if (work) std::copy(p->work.begin(), p->work.end(), work);
   return H3HIP_OK;
 }
 

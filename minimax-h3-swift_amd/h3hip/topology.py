@@ -119,7 +119,8 @@ def schedule(row_ptr: np.ndarray, heads: int, groups: int = 256):
     (h3hip_schedule): (work_ptr [groups + 1], work [heads * n_tiles]) int32;
     workgroup b runs work[work_ptr[b]:work_ptr[b + 1]], each unit
     head << 16 | q_tile. h3hip_plan_create uploads the same lists, or a list of half
-    units (64 queries) where few or uneven units make that end earlier."""
+    units (64 queries) where few or uneven units make that end earlier:
+    ``TilePlan.schedule`` gives a plan's own."""
     rp = np.ascontiguousarray(row_ptr, dtype=np.int32)
     n = len(rp) - 1
     work_ptr = np.zeros(groups + 1, dtype=np.int32)
@@ -174,6 +175,20 @@ class TilePlan:
         L.check(L.lib().h3hip_plan_tiles(self.handle, row_ptr.ctypes.data_as(i32p),
                                          col_idx.ctypes.data_as(i32p)))
         return row_ptr, col_idx[:self.nnz]
+
+    def schedule(self):
+        """The schedule this plan's launches run (h3hip_plan_schedule): (unit_rows,
+        work_ptr [groups + 1], work) int32, units of unit_rows queries (128 or
+        64), each head << 16 | row with row counting such query ranges."""
+        unit_rows, groups = ctypes.c_int32(), ctypes.c_int32()
+        fn = L.lib().h3hip_plan_schedule
+        L.check(fn(self.handle, ctypes.byref(unit_rows), ctypes.byref(groups), None, None))
+        work_ptr = np.zeros(groups.value + 1, dtype=np.int32)
+        work = np.zeros(self.heads * self.n_tiles * L.TILE // unit_rows.value, dtype=np.int32)
+        i32p = ctypes.POINTER(ctypes.c_int32)
+        L.check(fn(self.handle, None, None, work_ptr.ctypes.data_as(i32p),
+                   work.ctypes.data_as(i32p)))
+        return unit_rows.value, work_ptr, work
 
     @property
     def density(self) -> float:
