@@ -3,13 +3,15 @@
 // uneven to keep the CUs busy (plan creation decides, tile_plan.hip).
 //
 // A launch of few units is bound by one unit's serial chain: its tiles, each
-// with its loads' and LDS's latency, and its merge. Half a unit is 0.85 of a
-// tile per tile and half the merge (the LDS gives it its 128 KiB of operand
-// reads a tile in half the time; the loads are the same), and there are twice
-// as many. Measured on MI355X, full against half units: a band of 4,096 tokens x
-// 4 heads 14.1 -> 11.1 us, 917 dense tokens x 8 heads 15.6 -> 11.7 us, 5,372 x 2
-// heads 52.1 -> 41.7 us, and 31,885 local tokens x 2 heads, whose few prefix rows
-// see every tile, 292 -> 234 us. Each query's arithmetic is the same, in the same
+// with its loads' and LDS's latency, and its merge. Half a unit has a shorter
+// chain (the LDS gives it its 128 KiB of operand reads a tile in half the time;
+// the loads are the same), and there are twice as many. On an idle MI355X it takes
+// 0.80 us a tile against 1.07, and 5.4 us against 7.0 beyond its tiles, launch
+// included; where all CUs work, two half units take 1.13-1.28 times a whole one's
+// time. Measured, full against half units: a band of 4,096 tokens x 4 heads 14.1 ->
+// 11.1 us, 917 dense tokens x 8 heads 15.6-16.3 -> 11.7-12.2 us, 5,372 x 2 heads 52.1-53.4
+// -> 40.4-41.7 us, and 31,885 local tokens x 2 heads, whose few prefix rows see every
+// tile, 290-295 -> 234-237 us. Each query's arithmetic is the same, in the same
 // order: so are the bits. One wave per SIMD leaves the registers for eight loads
 // a tile; the tile loop is generated (gen_half_loop.py).
 #include "bsattn.h"

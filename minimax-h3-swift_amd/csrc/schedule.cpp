@@ -191,13 +191,19 @@ static int spread_units(int32_t heads, int32_t rows, int32_t groups,
   return check_units(heads, rows, work);
 }
 
-// Cost of a unit beyond its tiles and of a tile, in full units' tiles, where a
-// workgroup runs few units: dense rows of 8, 17 and 42 tiles, one unit each, take
-// 15.4, 25.1 and 52.2 us in full units and 11.3, 18.9 and 42.2 in half ones on MI355X,
-// launch included.
+// Cost of a unit beyond its tiles and of a tile, in whole units' tiles, for the
+// comparison below: a rule on the cautious side, not the cost of a half unit, which
+// depends on how busy the chip is. Alone on its CU a half unit takes 0.73-0.82 of a
+// whole one's time (dense rows of 3, 8, 16 and 42 tiles on MI355X: 7.8, 11.4, 17.4
+// and 38.9 us against 10.2, 15.4, 23.6 and 51.8, launch included); where all CUs
+// work, two take 1.13-1.28 of one (the constants say 1.7). Of 327 plans timed both
+// ways (equal, local, axial and drawn rows, 8 to 1,536 units) it picks the faster
+// units, or units within 0.5% of them, for 304. For 22 it stays with whole units
+// where half ones are up to 15% faster; one runs half units that are 3% slower.
 constexpr double kFullUnit = 2.0, kHalfUnit = 1.7, kHalfTile = 0.85;
-// Full units per workgroup up to which half units are looked at. Past it a
-// launch is bound by the chip's throughput, where half units cost 1.2-1.3 times.
+// Whole units per workgroup up to which half units are looked at. Past it a
+// launch is bound by the chip's throughput, where half units take 1.13-1.28 times
+// the whole ones' time.
 constexpr int kHalfUnitsUpTo = 6;
 
 // The time the cost model gives the longest workgroup of these lists.
