@@ -116,6 +116,18 @@ def test_named_sizes(pick):
     assert got == [c[0] for c in CASES], [(c, g) for c, g in zip(CASES, got) if c[0] != g]
 
 
+def test_sizes_of_the_eight_wave_tests(pick):
+    """What test_gpu_proj_eight_waves.py runs picks that kernel, and the row subsets
+    it compares with do not."""
+    import test_gpu_proj_eight_waves as t
+    whole = [(-(-S // 128) * 128, 384 * H, k, f) for S, k, H, *_ in t.QKV for f in (0, 1)]
+    whole += [(S, n, k, 0) for S, k, n, *_ in t.OUT]
+    parts = [(128, 384 * H, k, 0) for _, k, H, *_ in t.QKV] + [(t.ROWS, n, k, 0)
+                                                                for _, k, n, *_ in t.OUT]
+    assert pick(whole) == ["8wave"] * len(whole)
+    assert "8wave" not in pick(parts), pick(parts)
+
+
 def test_few_steps_take_small_tiles_only_for_one_round(pick):
     cases = [(t, n, h, f) for t in (1, 130, 700, 2000, 9000) for n in (256, 1536, 5120, 15360)
              for h in (64, 512, 960) for f in (0, 1)]
