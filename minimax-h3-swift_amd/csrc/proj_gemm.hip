@@ -1,6 +1,7 @@
 // The projections' GEMM on four waves: C = W x^T of h3hip_qkv_proj (with the
 // Q/K norm and RoPE in its epilogue, or plain) and of h3hip_out_proj, for every
-// size but short reductions (proj_tile.h).
+// size but short reductions that need more than one round of its smaller tiles
+// (proj_tile.h).
 //
 // What bounds it: at random bf16 operands the matrix cores run at the chip's
 // power limit, and between them and the operands stands the LDS, which gives

@@ -65,8 +65,8 @@ inline ProjGrid proj_grid(int tokens, int channels, int tile_tokens, int tile_ch
 // to an almost empty one's), over 64 sizes from 64 to 4,096 tokens of four layers:
 // the picks were the fastest shape or within 1.2% of it at 61 of them. Few
 // tiles are where it matters: 2,048 tokens x 5,120 channels are 160 tiles of 256
-// tokens (94 us) or 220 of 192 (87 us), 917 tokens 80 tiles (81 us), or 160 of 256 x
-// 128 (52 us) or 240 of 128 x 160 (42 us).
+// tokens (87-99 us) or 220 of 192 (80-82 us), 917 tokens 80 tiles (82 us), or 160 of
+// 256 x 128 (52 us) or 240 of 128 x 160 (42 us).
 //
 // With few reduction steps a tile is mostly its fill and epilogue: there the
 // eight-wave kernel, whose two waves per SIMD cover each other's epilogue, is

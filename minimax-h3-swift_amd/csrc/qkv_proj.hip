@@ -1,10 +1,10 @@
-// The projections' entry points and the eight-wave kernel, which runs the
-// reductions below 1,024 (1,536 with norm and RoPE): there a tile is mostly
-// fill and epilogue, and its two waves per SIMD cover each other's (18,102
-// tokens x 40 heads at hidden 512 with norm and RoPE: 361 us against 382 on four
-// waves). Longer reductions run the four-wave loop of proj_gemm.hip (31,885 x
-// 5,120 -> 15,360: 3.52 ms against 3.67 here); proj_tile.h picks, and both give
-// the same bits.
+// The projections' entry points and the eight-wave kernel. It runs reductions below
+// 1,024 (1,536 with norm and RoPE), where a tile is mostly fill and epilogue and
+// its two waves per SIMD cover each other's (18,102 tokens x 40 heads at hidden 512
+// with norm and RoPE: 361 us against 382 on four waves), except where one round of
+// a smaller four-wave tile does. Longer reductions run the four-wave loop of
+// proj_gemm.hip (31,885 x 5,120 -> 15,360: 3.52 ms against 3.67 here); proj_tile.h
+// picks, and both give the same bits.
 //
 // Fused QKV projection: the GEMM of AttentionLayer.callAsFunction
 // (Sources/H3Modules/DiTBlock.swift:336-338, `matmul(x, qkvWeight.T)` split

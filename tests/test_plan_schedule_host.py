@@ -128,3 +128,9 @@ def test_a_dropped_and_a_doubled_unit_are_refused(lib):
     assert lib.units_once(_p(work), 5, 2, 3) == 0
     work[5] = 0
     assert lib.units_once(_p(work), 6, 2, 3) == 0
+
+
+def test_no_plan_is_refused(h3):
+    from h3hip import _lib
+    assert h3.lib().h3hip_plan_schedule(None, None, None, None, None) == _lib.EINVAL
+    assert "plan is NULL" in h3.last_error()
